@@ -10,8 +10,8 @@ namespace artlite {
 // rows of A (tokens for gate / up, pairs for down) per decode tile
 constexpr int GEMV_BM = 4;
 
-// XQ, the decode activations: each row of K values (K a multiple of 256) as units of 256 values, a unit as 8
-// groups of 32 and each group as two int8 planes, x ~ s (a + b / 256) with s = max |x| / 127 over the group. A
+// XQ, the decode activations: each row of K values (K a multiple of 64) as units of 256 values (the last one's groups
+// past K are zeros), a unit as 8 groups of 32 and each group as two int8 planes, x ~ s (a + b / 256) with s = max |x| / 127 over the group. A
 // group's block is 16 dwords: plane a (8 dwords of 4 int8 in value order), then plane b. Per group three words:
 // s / 256 (fp32), the sum over the group of 256 a + b (int32), and s / 256 times that sum (fp32: the group's
 // dequantised sum). A group with a non-finite value has s = NaN; a group of zeros has s = 0.
@@ -20,7 +20,8 @@ constexpr int GEMV_BM = 4;
 // S = (dequantised sum of group 2 p, of group 2 p + 1)[r % 2]: chunk i is exactly what lane i of the GEMV needs.
 constexpr int XQ_UNIT = 256;  // dwords per unit
 
-__host__ __device__ inline int64_t xq_row_dwords(int K) { return int64_t(K / 256) * XQ_UNIT; }
+__host__ __device__ inline int xq_units(int K) { return (K + 255) / 256; }
+__host__ __device__ inline int64_t xq_row_dwords(int K) { return int64_t(xq_units(K)) * XQ_UNIT; }
 
 struct GemvArgs {
   const uint8_t* w[2];     // weight tensors: (gate, up) or (down, null); expert e at w + e expert_bytes
@@ -38,7 +39,8 @@ struct GemvArgs {
   const int32_t* offsets;  // E + 1 expert offsets in the sorted order
   int dense_rows;
   int64_t max_tiles;       // grid bound
-  uint32_t* hq;            // SwiGLU: h = silu(gate) up as XQ rows (by sorted row)
+  uint32_t* hq;            // SwiGLU: h = silu(gate) up as XQ rows (by sorted row); the groups past N of a row's last
+                           // unit are not written (the caller's zeros)
   float* y;                // plain: fp32 rows (by sorted row), stride N
   // (SwiGLU, optional) the routing done by the launch itself: when logits is given, every workgroup routes the T
   // tokens' (T, E) logits in its LDS (gemv_route_fits) and takes its items from that; workgroup 0 also stores ids,
@@ -56,13 +58,11 @@ struct GemvArgs {
 // whether a SwiGLU GEMV launch can route T tokens of E experts, top k, itself (GemvArgs::route)
 bool gemv_route_fits(int64_t T, int E, int k);
 
-// whether the GEMV takes N rows of K values of weights of this type
+// whether the GEMV takes N rows of K values of weights of this type: K whole units of 256 values, or (formats of
+// 32-value blocks) a multiple of 64, whose last unit is partly past the row's end; N whole items of 64 rows
 bool gemv_supported(int qtype, int K, int N);
 
 int launch_gemv(const GemvArgs& a, hipStream_t s);
-
-// x (T rows of K fp32 or bf16 values) -> XQ rows
-int launch_quant(const void* x, int x_dtype, int64_t T, int K, uint32_t* xq, hipStream_t s);
 
 // one XQ row back to fp32 (host side, for inspection)
 void xq_dequant_row(const uint32_t* row, int K, float* out);

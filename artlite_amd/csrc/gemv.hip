@@ -611,7 +611,7 @@ struct Stream {
     lane = threadIdx.x & 63, p = lane >> 4, r = lane & 15;
     rb = wv / S, ks = wv % S;
     my = slab + wv * (D * WCH + XCH);
-    const int U = a.K / 256;
+    const int U = xq_units(a.K);
     u0 = ks;  // (the wave's K-units: ks, ks + S, ...; the pair reads neighbouring units, which share lines, together)
     NVw = (U - ks + S - 1) / S * NM;
 #pragma unroll
@@ -685,15 +685,18 @@ __device__ __forceinline__ void wait_read(const Stream<QT, SWIGLU, D>& st, int n
   read_unit<QT, MX>(w, x, sw + st.o_w, sw + st.o_r, sw + st.o_s, sx);
 }
 
-// The dot products of one step: the lane's two groups of the unit w against the M rows of A's records x.
-template <int QT, int M>
-__device__ __forceinline__ void step_terms(const uint32_t (&w)[Unit<QT>::LW], const u32x4 (&x)[GEMV_BM], int p,
+// The dot products of one step: the lane's two groups of the unit w against the M rows of A's records x. RAG: a row's
+// last unit may be partly past its end; !on: the lane's groups are (its scales, then bytes of whatever follows the
+// row, taken as 0, as the records' are).
+template <int QT, int M, bool RAG>
+__device__ __forceinline__ void step_terms(const uint32_t (&w)[Unit<QT>::LW], const u32x4 (&x)[GEMV_BM], int p, bool on,
                                            float (&acc)[M]) {
   static_for<2>([&](auto hc) {
     constexpr int H = decltype(hc)::value;
     uint32_t q[8];
     float d, mn;
     codes<QT, H>(w, 2 * p + H, q, d, mn);
+    if constexpr (RAG) d = on ? d : 0.0f, mn = on ? mn : 0.0f;
 #pragma unroll
     for (int t = 0; t < M; t++) acc[t] = group_term<QT, H>(acc[t], x[t][H], x[t][2], x[t][3], q, d, mn);
   });
@@ -704,7 +707,7 @@ __device__ __forceinline__ void step_terms(const uint32_t (&w)[Unit<QT>::LW], co
 // the weights LA steps ahead, then waits for its own; at the start of each K-unit that wait also covers the
 // records, which are read into registers with the weights, and the next K-unit's are loaded into the freed slot.
 // Returns with the sums of the four lanes of a row in every lane.
-template <int QT, bool SWIGLU, int M, int D>
+template <int QT, bool SWIGLU, int M, int D, bool RAG>
 __device__ __forceinline__ void run_item(Stream<QT, SWIGLU, D>& st, const Item& cur, const Item& nxt, bool has_next,
                                          int gs, float (&out)[SWIGLU ? 2 : 1][GEMV_BM]) {
   using SS = Stream<QT, SWIGLU, D>;
@@ -715,7 +718,9 @@ __device__ __forceinline__ void run_item(Stream<QT, SWIGLU, D>& st, const Item& 
 #pragma unroll
     for (int t = 0; t < M; t++) acc[mx][t] = 0.0f;
   u32x4 xc[GEMV_BM];
+  const int pv = RAG ? (st.a.K % 256) / 64 : 0;  // (RAG: the lane rows p < pv hold groups of the last unit)
   for (int v0 = 0; v0 < st.NVw; v0 += NM) {
+    const bool on = !RAG || st.p < pv || st.u0 + SS::S * (v0 / NM) < st.a.K / 256;
     static_for<NM>([&](auto jc) {
       constexpr int MX = decltype(jc)::value;
       const int v = v0 + MX;
@@ -740,7 +745,7 @@ __device__ __forceinline__ void run_item(Stream<QT, SWIGLU, D>& st, const Item& 
       } else {
         wait_read<QT, SWIGLU, 0, D>(st, st.nl - st.wend[D - 1], sw, st.xbase, w, xc);
       }
-      step_terms<QT, M>(w, xc, st.p, acc[MX]);
+      step_terms<QT, M, RAG>(w, xc, st.p, on, acc[MX]);
     });
   }
 #pragma unroll
@@ -756,7 +761,7 @@ __device__ __forceinline__ void run_item(Stream<QT, SWIGLU, D>& st, const Item& 
 }
 
 // A persistent workgroup: items snake_item(blockIdx.x, j, gridDim.x) of (tile, block of 16 RB rows), tile-major.
-template <int QT, bool SWIGLU, int D>
+template <int QT, bool SWIGLU, int D, bool RAG>
 __global__ __launch_bounds__(Shape<SWIGLU>::THREADS) __attribute__((amdgpu_waves_per_eu(QT == ARTLITE_Q4_0 ? 4 : 2))) void k_gemv(
     const GemvArgs a) {
   using W = Shape<SWIGLU>;
@@ -842,10 +847,10 @@ __global__ __launch_bounds__(Shape<SWIGLU>::THREADS) __attribute__((amdgpu_waves
     if (has_next) nxt = get_item(tab, j + 1);
     float out[NM][GEMV_BM];
     switch (cur.m) {
-      case 1: run_item<QT, SWIGLU, 1, D>(st, cur, nxt, has_next, gs, out); break;
-      case 2: run_item<QT, SWIGLU, 2, D>(st, cur, nxt, has_next, gs, out); break;
-      case 3: run_item<QT, SWIGLU, 3, D>(st, cur, nxt, has_next, gs, out); break;
-      default: run_item<QT, SWIGLU, 4, D>(st, cur, nxt, has_next, gs, out); break;
+      case 1: run_item<QT, SWIGLU, 1, D, RAG>(st, cur, nxt, has_next, gs, out); break;
+      case 2: run_item<QT, SWIGLU, 2, D, RAG>(st, cur, nxt, has_next, gs, out); break;
+      case 3: run_item<QT, SWIGLU, 3, D, RAG>(st, cur, nxt, has_next, gs, out); break;
+      default: run_item<QT, SWIGLU, 4, D, RAG>(st, cur, nxt, has_next, gs, out); break;
     }
     gs += st.NVw;
     if constexpr (!SWIGLU) {
@@ -877,7 +882,7 @@ __global__ __launch_bounds__(Shape<SWIGLU>::THREADS) __attribute__((amdgpu_waves
           // lanes 8 RB / 2 t .. + 8 RB / 2 take row of A t: 8 lanes per XQ group of 32 rows, 4 rows each
           constexpr int LPT = 8 * RB / 2;
           const int t = ln / LPT, lt = ln % LPT, l8 = lt & 7, rbb = lt >> 2, r0 = 4 * (lt & 3);
-          const int UH = a.N / 256, blk = cur.n0 / 32 + (lt >> 3), g = blk & 7;
+          const int UH = xq_units(a.N), blk = cur.n0 / 32 + (lt >> 3), g = blk & 7;
           float4 gsum = {0.0f, 0.0f, 0.0f, 0.0f}, usum = gsum;
 #pragma unroll
           for (int k = 0; k < S; k++) {
@@ -913,13 +918,6 @@ __global__ __launch_bounds__(Shape<SWIGLU>::THREADS) __attribute__((amdgpu_waves
   }
 }
 
-// one wave per (row, unit) of x
-template <int XT>
-__global__ __launch_bounds__(256) void k_quant(const void* __restrict__ x, int64_t T, int K, uint32_t* __restrict__ xq) {
-  const int64_t w = (int64_t(blockIdx.x) * 256 + threadIdx.x) >> 6;
-  if (w < T * (K / 256)) xq_quant_unit<XT>(x, w, K, xq, threadIdx.x & 63);
-}
-
 // work items of a launch (the tile bound times the blocks of 16 RB rows)
 template <bool SWIGLU>
 int64_t gemv_items(const GemvArgs& a) {
@@ -928,14 +926,14 @@ int64_t gemv_items(const GemvArgs& a) {
   return tiles * ((a.N + 16 * W::RB - 1) / (16 * W::RB));
 }
 
-// persistent workgroups of k_gemv<QT, SWIGLU, D>: as many as the device holds at once (queried once per kernel, with
+// persistent workgroups of k_gemv<QT, SWIGLU, D, RAG>: as many as the device holds at once (queried once per kernel, with
 // a table of 64 items; 0: set-up failed); their item tables take 32 bytes an item, at most lds_max in all
-template <int QT, bool SWIGLU, int D>
+template <int QT, bool SWIGLU, int D, bool RAG>
 int gemv_resident() {
   using W = Shape<SWIGLU>;
   constexpr size_t lds0 = gemv_lds<QT, SWIGLU, D>(), lds_max = lds0 + 8192;
   static const int resident = [] {
-    const void* f = reinterpret_cast<const void*>(k_gemv<QT, SWIGLU, D>);
+    const void* f = reinterpret_cast<const void*>(k_gemv<QT, SWIGLU, D, RAG>);
     int dev = 0, cus = 0, per_cu = 0;
     if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds_max)) != hipSuccess ||
         hipGetDevice(&dev) != hipSuccess ||
@@ -947,14 +945,14 @@ int gemv_resident() {
   return resident;
 }
 
-template <int QT, bool SWIGLU, int D>
+template <int QT, bool SWIGLU, int D, bool RAG>
 int launch_t(const GemvArgs& a, hipStream_t s) {
   using W = Shape<SWIGLU>;
   const int64_t items = gemv_items<SWIGLU>(a);
   if (items <= 0) return ARTLITE_OK;
   if (items >= (int64_t(1) << 31)) return fail(ARTLITE_EINVAL, "expert GEMV: %lld work items", (long long)items);
   constexpr size_t lds0 = gemv_lds<QT, SWIGLU, D>(), lds_max = lds0 + 8192;
-  const int resident = gemv_resident<QT, SWIGLU, D>();
+  const int resident = gemv_resident<QT, SWIGLU, D, RAG>();
   if (resident <= 0) return fail(ARTLITE_EHIP, "expert GEMV: kernel set-up failed");
   const unsigned grid = unsigned(std::min<int64_t>(items, resident));
   const size_t lds = lds0 + size_t((items + grid - 1) / grid) * 32;
@@ -970,7 +968,7 @@ int launch_t(const GemvArgs& a, hipStream_t s) {
       return fail(ARTLITE_EINVAL, "expert GEMV: routing of %d tokens, %d experts, top %d in the launch", r.T, r.E,
                   r.k);
   }
-  k_gemv<QT, SWIGLU, D><<<grid, W::THREADS, lds, s>>>(a);
+  k_gemv<QT, SWIGLU, D, RAG><<<grid, W::THREADS, lds, s>>>(a);
   ART_HIP(hipGetLastError());
   return ARTLITE_OK;
 }
@@ -984,57 +982,56 @@ bool gemv_route_fits(int64_t T, int E, int k) {
          T * k <= Shape<true>::THREADS && T * E <= 8192;
 }
 
+namespace {
+// the formats of 32-value blocks (a row of any multiple of 64 values is whole blocks, and a whole number of dwords)
+bool gemv_blocks32(int qtype) {
+  return qtype == ARTLITE_Q4_0 || qtype == ARTLITE_Q8_0 || qtype == ARTLITE_Q4_1 || qtype == ARTLITE_IQ4_NL;
+}
+}  // namespace
+
 bool gemv_supported(int qtype, int K, int N) {
-  return (qtype == ARTLITE_Q4_0 || qtype == ARTLITE_Q8_0 || qtype == ARTLITE_Q4_K || qtype == ARTLITE_Q5_K ||
-          qtype == ARTLITE_Q6_K || qtype == ARTLITE_Q4_1 || qtype == ARTLITE_IQ4_NL || qtype == ARTLITE_IQ4_XS ||
-          qtype == ARTLITE_Q3_K) &&
-         K > 0 && K % 256 == 0 &&
-         N > 0 && N % 64 == 0;
+  const bool k256 = qtype == ARTLITE_Q4_K || qtype == ARTLITE_Q5_K || qtype == ARTLITE_Q6_K || qtype == ARTLITE_IQ4_XS ||
+                    qtype == ARTLITE_Q3_K;
+  return (gemv_blocks32(qtype) || k256) && K > 0 && K % (k256 ? 256 : 64) == 0 && N > 0 && N % 64 == 0;
 }
 
 int launch_gemv(const GemvArgs& a, hipStream_t s) {
   if (!gemv_supported(a.qtype, a.K, a.N))
     return fail(ARTLITE_EINVAL,
-                "expert GEMV: weight type %d with K %d, N %d (K a multiple of 256, N of 64)",
+                "expert GEMV: weight type %d with K %d, N %d (K a multiple of 256, or of 64 in 32-value blocks, N of 64)",
                 a.qtype, a.K, a.N);
   if (a.N <= 0 || int64_t(a.N) * a.row_bytes >= (int64_t(1) << 31))
     return fail(ARTLITE_EINVAL, "expert GEMV: %d rows of %d bytes", a.N, a.row_bytes);
   const bool swiglu = a.w[1] != nullptr;
-  if (swiglu && (a.N % 256 || !a.hq))
-    return fail(ARTLITE_EINVAL, "expert GEMV: SwiGLU width %d is not a multiple of 256", a.N);
+  if (swiglu && !a.hq) return fail(ARTLITE_EINVAL, "expert GEMV: no h");
   if (!swiglu && !a.y) return fail(ARTLITE_EINVAL, "expert GEMV: no output");
-#define ART_DISPATCH(QT) return swiglu ? launch_t<QT, true, WSLOTS>(a, s) : launch_t<QT, false, WSLOTS>(a, s)
+  // (a K of partial units: kernels of their own for the formats that have them, so that the others' steps are as
+  // they were)
+#define ART_DISPATCH(QT)                                                                                   \
+  return swiglu ? launch_t<QT, true, WSLOTS, false>(a, s) : launch_t<QT, false, WSLOTS, false>(a, s)
+#define ART_DISPATCH_32(QT)                                                                                \
+  if (a.K % 256)                                                                                           \
+    return swiglu ? launch_t<QT, true, WSLOTS, true>(a, s) : launch_t<QT, false, WSLOTS, true>(a, s);      \
+  ART_DISPATCH(QT)
   switch (a.qtype) {
-    case ARTLITE_Q4_0: ART_DISPATCH(ARTLITE_Q4_0);
-    case ARTLITE_Q8_0: ART_DISPATCH(ARTLITE_Q8_0);
+    case ARTLITE_Q4_0: ART_DISPATCH_32(ARTLITE_Q4_0);
+    case ARTLITE_Q8_0: ART_DISPATCH_32(ARTLITE_Q8_0);
+    case ARTLITE_Q4_1: ART_DISPATCH_32(ARTLITE_Q4_1);
+    case ARTLITE_IQ4_NL: ART_DISPATCH_32(ARTLITE_IQ4_NL);
     case ARTLITE_Q5_K: ART_DISPATCH(ARTLITE_Q5_K);
     case ARTLITE_Q6_K: ART_DISPATCH(ARTLITE_Q6_K);
     case ARTLITE_Q3_K: ART_DISPATCH(ARTLITE_Q3_K);
-    case ARTLITE_Q4_1: ART_DISPATCH(ARTLITE_Q4_1);
-    case ARTLITE_IQ4_NL: ART_DISPATCH(ARTLITE_IQ4_NL);
     case ARTLITE_IQ4_XS: ART_DISPATCH(ARTLITE_IQ4_XS);
     default: ART_DISPATCH(ARTLITE_Q4_K);
   }
+#undef ART_DISPATCH_32
 #undef ART_DISPATCH
 }
 
-int launch_quant(const void* x, int x_dtype, int64_t T, int K, uint32_t* xq, hipStream_t s) {
-  if (T <= 0) return ARTLITE_OK;
-  if (K <= 0 || K % 256) return fail(ARTLITE_EINVAL, "quant: K %d is not a multiple of 256", K);
-  const int64_t waves = T * (K / 256);
-  const unsigned blocks = unsigned((waves + 3) / 4);
-  if (x_dtype == ARTLITE_X_F32)
-    k_quant<ARTLITE_X_F32><<<blocks, 256, 0, s>>>(x, T, K, xq);
-  else
-    k_quant<ARTLITE_X_BF16><<<blocks, 256, 0, s>>>(x, T, K, xq);
-  ART_HIP(hipGetLastError());
-  return ARTLITE_OK;
-}
-
 void xq_dequant_row(const uint32_t* row, int K, float* out) {
-  for (int u = 0; u < K / 256; u++) {
+  for (int u = 0; u < xq_units(K); u++) {
     const uint32_t* ub = row + int64_t(u) * XQ_UNIT;
-    for (int g = 0; g < 8; g++) {
+    for (int g = 0; g < 8 && 256 * u + 32 * g < K; g++) {
       float s;
       std::memcpy(&s, &ub[4 * (16 * (g >> 1) + 2 * (g & 1)) + 2], 4);
       for (int v = 0; v < 32; v++) {

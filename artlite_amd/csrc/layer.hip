@@ -2,6 +2,7 @@
 // forward pass on one HIP stream: router -> top k -> dispatch -> gate / up (SwiGLU) -> down -> combine, plus the
 // shared expert. The semantics are the reference's oracle (tests/moe/ref.py:43-60) with its routing
 // (csrc/artlite/moe_host.cpp:45-73) and combine (src/artlite/moe/gather.py:12-18).
+#include <algorithm>
 #include <cmath>
 #include <string>
 #include <vector>
@@ -41,7 +42,7 @@ struct artlite_moe_layer {
   DevBuf pq_gate, pq_up, pq_down, pq_sgate, pq_sup, pq_sdown;
   int pre_g = 0, pre_d = 0, pre_sg = 0, pre_sd = 0;  // the prefill launches' weight format of each product (0: none)
   DevBuf xq, hq, shq;  // the decode path's XQ activations
-  bool gemv_ok = false, shared_gemv_ok = false, prefill_ok = false, shared_prefill_ok = false;
+  bool gemv_ok = false, shared_gemv_ok = false /* beside routed experts on the GEMV */, prefill_ok = false, shared_prefill_ok = false;
   int64_t last_T = -1;
   bool last_gemv = false, last_prefill = false;
   int last_ys_parts = 1;  // (the shared expert's output of the last run: parts of its K, summed by the combine)
@@ -141,7 +142,9 @@ int check_ready(const artlite_moe_layer* L) {
 // average) run the experts on the VALU GEMV over XQ activations (it takes every block format); larger ones on the
 // fp16 MFMA prefill tiles (every block format: Q4_0, Q8_0, Q4_K from the file's bytes, the others through the prefill
 // layout), and where those do not take a product's shape (K below 320 or not a multiple of 64) on the MFMA decode
-// tiles over bf16 planes. (At 128 tokens of config 2, 8 pairs per expert, the prefill tiles' tiles of 32 rows took
+// tiles over bf16 planes. (The GEMV takes widths of partial units in the formats of 32-value blocks: at 8 tokens of 64
+// experts 1408 wide the routed experts took 183 us on the prefill tiles, whose steps are as long for two rows of a tile
+// as for 32, and 47 us on the GEMV; at 5 tokens of 32 experts 2880 wide the layer 215 against 91 us.) (At 128 tokens of config 2, 8 pairs per expert, the prefill tiles' tiles of 32 rows took
 // 208 us against 323 on the MFMA decode tiles: the decode tiles do twice the MFMA work on bf16 hi / lo planes.)
 struct Path {
   bool gemv;            // routed experts (gate / up and down) on the GEMV (XQ of x; tiles of GEMV_BM rows)
@@ -608,7 +611,7 @@ extern "C" int artlite_moe_layer_create(const artlite_moe_desc* desc, artlite_mo
     L->sgate_row = size_t(d.hidden) / sq->per * sq->dev;
     L->sdown_row = size_t(d.shared_ffn) / sdq->per * sdq->dev;
   }
-  L->gemv_ok = gemv_supported(d.gate_type, d.hidden, d.expert_ffn) && d.expert_ffn % 256 == 0 &&
+  L->gemv_ok = gemv_supported(d.gate_type, d.hidden, d.expert_ffn) &&
                gemv_supported(d.down_type, d.expert_ffn, d.hidden);
   // (the prefill tiles address weights and A rows by 32-bit offsets: every expert's bytes, every row of x16 and h16)
   const int64_t maxP = int64_t(d.max_tokens) * d.top_k;
@@ -620,7 +623,10 @@ extern "C" int artlite_moe_layer_create(const artlite_moe_desc* desc, artlite_mo
                                d.max_tokens, d.hidden) &&
                   prefill_fits(d.n_experts, int64_t(d.hidden) * prefill_row(L->down_row, d.expert_ffn, L->pre_d), maxP,
                                d.expert_ffn);
-  L->shared_gemv_ok = sq && gemv_supported(sq->id, d.hidden, d.shared_ffn) &&
+  // (a shared expert beside routed ones of a partial unit stays on the MFMA decode tiles: its bf16 hi / lo planes hold
+  // x and h to 2^-17, XQ to 2^-16 of a group's largest, and its output is the layer's largest term)
+  L->shared_gemv_ok = sq && d.hidden % 256 == 0 && d.expert_ffn % 256 == 0 && d.shared_ffn % 256 == 0 &&
+                      gemv_supported(sq->id, d.hidden, d.shared_ffn) &&
                       gemv_supported(sdq->id, d.shared_ffn, d.hidden);
   L->pre_sg = prefill_type(sq);
   L->pre_sd = prefill_type(sdq);
@@ -680,17 +686,25 @@ extern "C" int artlite_moe_layer_create(const artlite_moe_desc* desc, artlite_mo
     }
   }
   if (L->gemv_ok) {
-    res(L->xq, size_t(T * xq_row_dwords(d.hidden)) * 4);
-    res(L->hq, size_t(P * xq_row_dwords(d.expert_ffn)) * 4);
-    if (L->shared_gemv_ok) res(L->shq, size_t(T * xq_row_dwords(d.shared_ffn)) * 4);
+    // (the passes path_of gives the GEMV: at most GEMV_BM pairs per expert on average)
+    const int64_t gP = std::min<int64_t>(P, GEMV_BM * E), gT = std::min<int64_t>(T, GEMV_BM * E / d.top_k);
+    res(L->xq, size_t(gT * xq_row_dwords(d.hidden)) * 4);
+    res(L->hq, size_t(gP * xq_row_dwords(d.expert_ffn)) * 4);
+    if (L->shared_gemv_ok) res(L->shq, size_t(gT * xq_row_dwords(d.shared_ffn)) * 4);
   }
   if (d.shared_ffn) {
     res(L->shhi, size_t(T) * d.shared_ffn * 2);
     res(L->shlo, size_t(T) * d.shared_ffn * 2);
     res(L->ys, size_t(T * H) * 4 * (L->shared_prefill_ok ? PREFILL_MAXP : 1));  // (prefill: the down's K parts)
   }
-  if (rc == ARTLITE_OK && hipMemset(L->ctrl.p, 0, CTRL_WORDS * 4) != hipSuccess)
-    rc = fail(ARTLITE_EHIP, "moe layer: memset");
+  // (h in XQ rows of a width of partial units: the groups past it, zeros that no launch writes)
+  auto zero = [&](const DevBuf& b, size_t bytes) {
+    if (rc == ARTLITE_OK && b.p && hipMemsetAsync(b.p, 0, bytes, L->stream) != hipSuccess)
+      rc = fail(ARTLITE_EHIP, "moe layer: memset");
+  };
+  zero(L->ctrl, CTRL_WORDS * 4);
+  if (F % 256) zero(L->hq, L->hq.n);
+  if (rc == ARTLITE_OK && hipStreamSynchronize(L->stream) != hipSuccess) rc = fail(ARTLITE_EHIP, "moe layer: memset");
   if (rc != ARTLITE_OK) {
     artlite_moe_layer_destroy(L);
     return rc;

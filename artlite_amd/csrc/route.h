@@ -267,7 +267,7 @@ int launch_topk_parts(const double* part, int parts, int64_t n, int E, float* ou
                       int32_t* ids, float* w32, hipStream_t s);
 
 // Router logits out[t out_row + e] = x[t] . W[e] (float64 accumulation, rounded once). xq: when given, x is also
-// quantised into XQ rows (gemv.h) by extra workgroups of the same launch (H a multiple of 256). part (part_elems
+// quantised into XQ rows (gemv.h) by extra workgroups of the same launch (H a multiple of 64). part (part_elems
 // doubles, router_part_elems for the most tokens of a layer; may be null): the fp64 partial sums of prefill-sized
 // batches whose tiles are too few for the device, K split over workgroups and the parts added in a fixed order.
 // parts_left (optional): the parts are then not added here: *parts_left = their count (for launch_topk_parts), or 0
@@ -621,7 +621,7 @@ int launch_route_small(const float* logits, int64_t n, int E, int k, int sigmoid
                        const DispatchBufs& d, hipStream_t s);
 
 // Router logits (as launch_router, into logits (T, E)) of small batches: T <= ROUTER_GROUPS ROUTER_TG tokens, H a
-// multiple of 256 (at least 2 values per wave), E <= MAX_EXPERTS (router_few_fits). xq: when given, x is also
+// multiple of 32, E <= MAX_EXPERTS (router_few_fits). xq: when given, x is also
 // quantised into XQ rows.
 bool router_few_fits(int64_t T, int H, int E);
 int launch_router_few(const void* x, int x_dtype, const float* W, int H, int E, int64_t T, float* logits,

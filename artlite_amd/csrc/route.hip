@@ -118,7 +118,7 @@ __global__ __launch_bounds__(EW * WAVE) void k_router(const void* __restrict__ x
   if (int(blockIdx.x) >= nbx) {  // XQ of x
     if (blockIdx.y) return;
     const int64_t w = int64_t(blockIdx.x - nbx) * EW + wv;
-    if (w < T * (H / 256)) xq_quant_unit<XT>(xv, w, H, xq, lane);
+    if (w < T * xq_units(H)) xq_quant_unit<XT>(xv, w, H, xq, lane);
     return;
   }
   const int64_t t0 = int64_t(blockIdx.y) * tt;
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(4 * WAVE) void k_router_small(const void* __restric
   if (int(blockIdx.x) >= E) {  // XQ of x
     if (blockIdx.y) return;
     const int64_t w = int64_t(blockIdx.x - E) * 4 + wv;
-    if (w < T * (H / 256)) xq_quant_unit<XT>(xv, w, H, xq, lane);
+    if (w < T * xq_units(H)) xq_quant_unit<XT>(xv, w, H, xq, lane);
     return;
   }
   const int e = blockIdx.x;
@@ -500,7 +500,7 @@ int launch_router(const void* x, int x_dtype, const float* W, int H, int E, int6
   if (parts_left) *parts_left = 0;
   if (T <= 0) return ARTLITE_OK;
   if (H % 8) return fail(ARTLITE_EINVAL, "router: H %d not a multiple of 8", H);
-  if (xq && H % 256) return fail(ARTLITE_EINVAL, "router: XQ of H %d (not a multiple of 256)", H);
+  if (xq && H % 64) return fail(ARTLITE_EINVAL, "router: XQ of H %d (not a multiple of 64)", H);
   const int xb = x_dtype == ARTLITE_X_F32 ? 4 : 2;
   const int tt = int(std::min<int64_t>(ROUTER_TG, std::max<int64_t>(1, ROUTER_LDS / (int64_t(H) * xb))));
   if (int64_t(H) * xb > ROUTER_LDS) return fail(ARTLITE_EINVAL, "router: H %d too wide", H);
@@ -537,7 +537,7 @@ int launch_router(const void* x, int x_dtype, const float* W, int H, int E, int6
     return ARTLITE_OK;
   }
   if (T <= ROUTER_TG && H % 1024 == 0) {  // (a workgroup per expert)
-    const int nq = xq ? int((T * (H / 256) + 3) / 4) : 0;
+    const int nq = xq ? int((T * xq_units(H) + 3) / 4) : 0;
     const dim3 g(unsigned(E + nq), 1), b(4 * WAVE);
     if (x_dtype == ARTLITE_X_F32)
       k_router_small<ARTLITE_X_F32><<<g, b, 0, s>>>(x, W, H, E, T, out, out_row, xq);
@@ -550,7 +550,7 @@ int launch_router(const void* x, int x_dtype, const float* W, int H, int E, int6
   const bool small = T <= 4 * ROUTER_TG;
   const int ew = small ? 4 : ROUTER_EW;
   const int nbx = (E + ew - 1) / ew;
-  const int nq = xq ? int((T * (H / 256) + ew - 1) / ew) : 0;
+  const int nq = xq ? int((T * xq_units(H) + ew - 1) / ew) : 0;
   const dim3 grid(unsigned(nbx + nq), unsigned((T + tt - 1) / tt)), block(ew * WAVE);
 #define ART_ROUTER(XT, EWN) k_router<XT, EWN><<<grid, block, lds, s>>>(x, W, H, E, T, tt, out, out_row, xq, nbx)
   if (x_dtype == ARTLITE_X_F32) {
@@ -580,7 +580,7 @@ __global__ __launch_bounds__(DISPATCH_BLOCK) void k_route_small(const float* __r
   route_core<DISPATCH_BLOCK, R>(logits, int(n), E, k, sigmoid, d.BM, d.balanced, ids, w32, d, true, lds, RouteOut{});
 }
 
-// Router logits of small batches (T <= ROUTER_GROUPS ROUTER_TG tokens, H a multiple of 256, at least 2 values a
+// Router logits of small batches (T <= ROUTER_GROUPS ROUTER_TG tokens, H a multiple of 32: an even number of values a
 // wave). A workgroup per EPW experts and group of ROUTER_TG tokens (workgroup b: experts EPW (b % (E / EPW)) .., tokens
 // ROUTER_TG (b / (E / EPW)) ..): each expert's NW / EPW waves each take a slice of H / (NW / EPW) values of K (lane:
 // values 2 lane + 128 j of the wave's slice), x read straight from memory (L2), float64 products; a wave's 16 token
@@ -597,7 +597,7 @@ __global__ __launch_bounds__(DISPATCH_BLOCK) void k_router_few(const void* __res
   const int G = int((T + ROUTER_TG - 1) / ROUTER_TG), EB = E / EPW;  // (token groups, expert blocks)
   if (int(blockIdx.x) >= EB * G) {  // XQ of x
     const int64_t w = int64_t(blockIdx.x - EB * G) * NW + wv;
-    if (w < T * (H / 256)) xq_quant_unit<XT>(xv, w, H, xq, lane);
+    if (w < T * xq_units(H)) xq_quant_unit<XT>(xv, w, H, xq, lane);
     return;
   }
   const int eb = int(blockIdx.x) % EB, gi = int(blockIdx.x) / EB, t0 = gi * ROUTER_TG, nt = min(ROUTER_TG, int(T) - t0);
@@ -676,7 +676,7 @@ int launch_route_small(const float* logits, int64_t n, int E, int k, int sigmoid
 }
 
 bool router_few_fits(int64_t T, int H, int E) {
-  return T >= 1 && T <= ROUTER_GROUPS * ROUTER_TG && H % 256 == 0 && H / (DISPATCH_BLOCK / WAVE) >= 2 &&
+  return T >= 1 && T <= ROUTER_GROUPS * ROUTER_TG && H % (2 * (DISPATCH_BLOCK / WAVE)) == 0 && H > 0 &&
          E <= MAX_EXPERTS;
 }
 
@@ -685,7 +685,7 @@ int launch_router_few(const void* x, int x_dtype, const float* W, int H, int E, 
   if (!router_few_fits(T, H, E))
     return fail(ARTLITE_EINVAL, "router_few: %lld tokens, H %d, %d experts", (long long)T, H, E);
   constexpr int NW = DISPATCH_BLOCK / WAVE;
-  const int nq = xq ? int((T * (H / 256) + NW - 1) / NW) : 0;
+  const int nq = xq ? int((T * xq_units(H) + NW - 1) / NW) : 0;
   // (past two token groups, two experts a workgroup: fewer, longer workgroups, which the device holds in one round)
   const int epw = T > 2 * ROUTER_TG && E % 2 == 0 ? 2 : 1;
   const dim3 g(unsigned(E / epw * ((T + ROUTER_TG - 1) / ROUTER_TG) + nq)), b(DISPATCH_BLOCK);

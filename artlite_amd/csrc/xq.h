@@ -75,16 +75,17 @@ __device__ __forceinline__ void xq_put_word(uint32_t* ub, int g, int k, float s2
 }
 
 // One unit (256 values) of row `row` of x (T rows of K fp32 / bf16 values; XT its dtype) into XQ, by one wave: lane
-// l quantises values 4 l .. 4 l + 3 (group l / 8, plane dword l % 8). w: the wave's (row, unit) index.
+// l quantises values 4 l .. 4 l + 3 (group l / 8, plane dword l % 8; past K: zeros). w: the wave's (row, unit) index.
 template <int XT>
 __device__ __forceinline__ void xq_quant_unit(const void* __restrict__ x, int64_t w, int K, uint32_t* __restrict__ xq,
                                               int lane) {
-  const int U = K / 256;
+  const int U = xq_units(K);
   const int64_t row = w / U;
   const int u = int(w - row * U);
   const int64_t i0 = row * K + int64_t(u) * 256 + 4 * lane;
-  float v[4];
-  if (XT == ARTLITE_X_F32) {
+  float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (u * 256 + 4 * lane >= K) {
+  } else if (XT == ARTLITE_X_F32) {
     const float4 f = *reinterpret_cast<const float4*>(static_cast<const float*>(x) + i0);
     v[0] = f.x, v[1] = f.y, v[2] = f.z, v[3] = f.w;
   } else {
