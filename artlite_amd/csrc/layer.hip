@@ -10,6 +10,7 @@
 #include "experts.h"
 #include "gemv.h"
 #include "route.h"
+#include "stream.h"
 
 using namespace artlite;
 
@@ -42,6 +43,7 @@ struct artlite_moe_layer {
   DevBuf pq_gate, pq_up, pq_down, pq_sgate, pq_sup, pq_sdown;
   int pre_g = 0, pre_d = 0, pre_sg = 0, pre_sd = 0;  // the prefill launches' weight format of each product (0: none)
   DevBuf xq, hq, shq;  // the decode path's XQ activations
+  bool stream_ok = false /* routed, beside prefill_ok */, shared_stream_ok = false;
   bool gemv_ok = false, shared_gemv_ok = false /* beside routed experts on the GEMV */, prefill_ok = false, shared_prefill_ok = false;
   int64_t last_T = -1;
   bool last_gemv = false, last_prefill = false;
@@ -146,11 +148,20 @@ int check_ready(const artlite_moe_layer* L) {
 // experts 1408 wide the routed experts took 183 us on the prefill tiles, whose steps are as long for two rows of a tile
 // as for 32, and 47 us on the GEMV; at 5 tokens of 32 experts 2880 wide the layer 215 against 91 us.) (At 128 tokens of config 2, 8 pairs per expert, the prefill tiles' tiles of 32 rows took
 // 208 us against 323 on the MFMA decode tiles: the decode tiles do twice the MFMA work on bf16 hi / lo planes.)
+// The prefill's routed products by the streamed small tiles (stream.hip): up to this many pairs per expert on average in
+// tiles of 16 rows, then of 32, then no longer. Layer times of the 128-expert Q4_0 layer at 200 / 256 / 400 / 512 / 700
+// tokens (12.5 / 16 / 25 / 32 / 44 pairs): tiles of 16 129 / 148 / 196 / 228 / 290 us, of 32 142 / 146 / 161 / 193 /
+// 246 us, the MFMA prefill tiles 208 / 206 / 211 / 215 / 231 us. A shared expert of the routed format joins the prefill
+// tiles' launches and not these (64 experts of Q4_K, 24 / 48 pairs: 268 / 347 against 294 / 302 us), so the line is lower.
+constexpr int STREAM_16 = 14, STREAM_32 = 38, STREAM_32_SHARED = 30;
+
 struct Path {
   bool gemv;            // routed experts (gate / up and down) on the GEMV (XQ of x; tiles of GEMV_BM rows)
   bool shared_gemv;     // the shared expert on the GEMV
   bool prefill;         // routed experts on the prefill tiles
+  int stream;           // ... their products by the streamed small tiles: their rows (16 or 32), 0: not
   bool shared_prefill;  // the shared expert on the prefill tiles
+  bool shared_stream;   // the shared expert on the streamed small tiles (bf16 planes)
   bool split;           // bf16 hi / lo planes of fp32 x needed (the MFMA decode tiles)
   bool quant;           // XQ of x needed (made by the router's launch)
   bool few_router;      // the router's launch of few tokens: a workgroup per expert and 16 tokens (and XQ of x)
@@ -164,6 +175,15 @@ Path path_of(const artlite_moe_layer* L, int64_t T) {
   p.shared_gemv = L->d.shared_ffn && p.gemv && L->shared_gemv_ok;
   p.prefill = !p.gemv && L->prefill_ok;
   p.shared_prefill = L->d.shared_ffn && p.prefill && L->shared_prefill_ok && T >= 64;
+  const int64_t P = T * L->d.top_k, E = L->d.n_experts;
+  const bool joins = L->shared_prefill_ok && (L->sq->id == L->gq->id || L->sdq->id == L->dq->id);
+  if (p.prefill && L->stream_ok && P <= int64_t(joins ? STREAM_32_SHARED : STREAM_32) * E) {
+    const int bm = P <= STREAM_16 * E ? 16 : 32;
+    if (stream_fits(L->d.gate_type, true, L->d.expert_ffn, bm, tile_bound(P, int(E), bm)) &&
+        stream_fits(L->d.down_type, false, L->d.hidden, bm, tile_bound(P, int(E), bm)))
+      p.stream = bm;
+  }
+  p.shared_stream = L->d.shared_ffn && !p.shared_gemv && !p.shared_prefill && L->shared_stream_ok;
   const bool planes = (!p.gemv && !p.prefill) || (L->d.shared_ffn && !p.shared_gemv && !p.shared_prefill);
   p.split = planes && (L->x_dtype == ARTLITE_X_F32 || L->d.norm_eps > 0);  // (the normalised x is fp32)
   p.quant = p.gemv;
@@ -174,9 +194,13 @@ Path path_of(const artlite_moe_layer* L, int64_t T) {
 }
 
 // whether the shared expert's gate / up (down) products join the routed launch on the prefill tiles: the same block
-// format (the launch's kernel is instantiated per format)
-bool shared_gu_merged(const artlite_moe_layer* L) { return L->sq && L->sq->id == L->gq->id; }
-bool shared_dn_merged(const artlite_moe_layer* L) { return L->sdq && L->sdq->id == L->dq->id; }
+// format (the launch's kernel is instantiated per format), and routed experts on those tiles
+bool shared_gu_merged(const artlite_moe_layer* L, const Path& p) {
+  return !p.stream && L->sq && L->sq->id == L->gq->id;
+}
+bool shared_dn_merged(const artlite_moe_layer* L, const Path& p) {
+  return !p.stream && L->sdq && L->sdq->id == L->dq->id;
+}
 
 // the named kernels of a forward pass, in launch order
 std::vector<std::string> kernel_list(const artlite_moe_layer* L, int64_t T) {
@@ -197,9 +221,9 @@ std::vector<std::string> kernel_list(const artlite_moe_layer* L, int64_t T) {
   }
   const bool sp = p.prefill && p.shared_prefill;  // (the shared expert's items in the routed launches, or beside them)
   k.push_back("gate_up");
-  if (sp && !shared_gu_merged(L)) k.push_back("shared_gate_up");
+  if (sp && !shared_gu_merged(L, p)) k.push_back("shared_gate_up");
   k.push_back("down");
-  if (sp && !shared_dn_merged(L)) k.push_back("shared_down");
+  if (sp && !shared_dn_merged(L, p)) k.push_back("shared_down");
   if (L->d.shared_ffn && !sp) {
     k.push_back("shared_gate_up");
     k.push_back("shared_down");
@@ -239,6 +263,30 @@ PrefillProblem shared_down_part(const artlite_moe_layer* L, int64_t T, int j, in
   return p;
 }
 
+// a routed product of the prefill on the streamed small tiles: the same operands, the weights from the file's bytes
+StreamArgs stream_of(const PrefillProblem& p, int qtype, const uint8_t* w0, const uint8_t* w1, size_t row, int bm,
+                     int64_t P) {
+  StreamArgs a{};
+  a.w[0] = w0;
+  a.w[1] = w1;
+  a.row_bytes = int(row);
+  a.expert_bytes = int64_t(p.N) * int64_t(row);
+  a.N = p.N;
+  a.K = p.K;
+  a.qtype = qtype;
+  a.a = p.a;
+  a.row_a = p.row_a;
+  a.row_scale = p.row_scale;
+  a.tiles = p.tiles;
+  a.n_tiles = p.n_tiles;
+  a.max_tiles = p.max_tiles;
+  a.rows = int(P);
+  a.bm = bm;
+  a.h = p.h;
+  a.y16 = p.y16;
+  return a;
+}
+
 // The forward pass of the staged T tokens. ev (optional): an event recorded before each kernel and one after the
 // last (kernel_list order).
 int run(artlite_moe_layer* L, int64_t T, hipEvent_t* ev) {
@@ -275,10 +323,10 @@ int run(artlite_moe_layer* L, int64_t T, hipEvent_t* ev) {
     ahi = L->xhi.as<uint16_t>();
     alo = L->xlo.as<uint16_t>();
   }
-  const int BM = path.gemv ? GEMV_BM : path.prefill ? PREFILL_BM : DECODE_BM;
+  const int BM = path.gemv ? GEMV_BM : path.stream ? path.stream : path.prefill ? PREFILL_BM : DECODE_BM;
   DispatchBufs db{L->ids.as<int32_t>(), P, E, k, L->table.as<int32_t>(), L->ctrl.as<int32_t>(),
                   L->counts.as<int32_t>(), L->offsets.as<int32_t>(), L->order.as<int32_t>(), L->slot.as<int32_t>(),
-                  L->tiles.as<int32_t>(), BM, nullptr, 0, path.prefill ? 1 : 0};
+                  L->tiles.as<int32_t>(), BM, nullptr, 0, path.prefill && !path.stream ? 1 : 0};
   if (path.prefill) {  // (the scatter also writes each sorted row's token and factors)
     db.row_a = L->row_a.as<int32_t>();
     db.row_f[0] = L->gu_tok.as<float2>();
@@ -391,7 +439,7 @@ int run(artlite_moe_layer* L, int64_t T, hipEvent_t* ev) {
     g.h = L->h16.as<uint16_t>();
     PrefillArgs sgu{};  // (the shared gate / up: in gu, or a launch of its own)
     if (sp) {
-      PrefillArgs& into = shared_gu_merged(L) ? gu : sgu;
+      PrefillArgs& into = shared_gu_merged(L, path) ? gu : sgu;
       prefill_format(L->sq, into);
       PrefillProblem& q = into.p[into.np++];
       q.w[0] = prefill_w(L->sgate, L->pq_sgate, L->pre_sg);
@@ -406,7 +454,10 @@ int run(artlite_moe_layer* L, int64_t T, hipEvent_t* ev) {
       q.h = L->sh16.as<uint16_t>();
     }
     ART_TRY(mark());
-    ART_TRY(launch_prefill(gu, s));
+    if (path.stream)
+      ART_TRY(launch_stream(stream_of(g, d.gate_type, L->gate.as<uint8_t>(), L->up.as<uint8_t>(), L->gate_row, path.stream, P), s));
+    else
+      ART_TRY(launch_prefill(gu, s));
     if (sgu.np) {
       ART_TRY(mark());
       ART_TRY(launch_prefill(sgu, s));
@@ -430,7 +481,7 @@ int run(artlite_moe_layer* L, int64_t T, hipEvent_t* ev) {
     q.y16 = L->ypairs.as<uint16_t>();  // (fp16 pair outputs, their rows' true values dn_row[s].x times these)
     PrefillArgs sdn{};  // (the shared down's parts: in dn, or a launch of their own)
     if (sp) {
-      const bool merged = shared_dn_merged(L);
+      const bool merged = shared_dn_merged(L, path);
       PrefillArgs& into = merged ? dn : sdn;
       prefill_format(L->sdq, into);
       const int n = shared_parts(L, merged);
@@ -444,7 +495,10 @@ int run(artlite_moe_layer* L, int64_t T, hipEvent_t* ev) {
       ys_parts = n;
     }
     ART_TRY(mark());
-    ART_TRY(launch_prefill(dn, s));
+    if (path.stream)
+      ART_TRY(launch_stream(stream_of(q, d.down_type, L->down.as<uint8_t>(), nullptr, L->down_row, path.stream, P), s));
+    else
+      ART_TRY(launch_prefill(dn, s));
     if (sdn.np) {
       ART_TRY(mark());
       ART_TRY(launch_prefill(sdn, s));
@@ -515,6 +569,34 @@ int run(artlite_moe_layer* L, int64_t T, hipEvent_t* ev) {
     ART_TRY(launch_gemv(sd, s));
     ys = L->ys.as<float>();
   } else if (d.shared_ffn && path.shared_prefill) {  // (with the routed experts' launches)
+    ys = L->ys.as<float>();
+  } else if (d.shared_ffn && path.shared_stream) {
+    StreamFewArgs sg{};
+    sg.w[0] = L->sgate.as<uint8_t>();
+    sg.w[1] = L->sup.as<uint8_t>();
+    sg.row_bytes = int(L->sgate_row);
+    sg.N = d.shared_ffn;
+    sg.K = H;
+    sg.qtype = d.shared_type;
+    sg.a = ahi;
+    sg.a_lo = alo;
+    sg.rows = int(T);
+    sg.h_hi = L->shhi.as<uint16_t>();
+    sg.h_lo = L->shlo.as<uint16_t>();
+    ART_TRY(mark());
+    ART_TRY(launch_stream_few(sg, s));
+    StreamFewArgs sd{};
+    sd.w[0] = L->sdown.as<uint8_t>();
+    sd.row_bytes = int(L->sdown_row);
+    sd.N = H;
+    sd.K = d.shared_ffn;
+    sd.qtype = L->sdq->id;
+    sd.a = L->shhi.as<uint16_t>();
+    sd.a_lo = L->shlo.as<uint16_t>();
+    sd.rows = int(T);
+    sd.y = L->ys.as<float>();
+    ART_TRY(mark());
+    ART_TRY(launch_stream_few(sd, s));
     ys = L->ys.as<float>();
   } else if (d.shared_ffn) {
     GemmArgs sg{};
@@ -628,6 +710,10 @@ extern "C" int artlite_moe_layer_create(const artlite_moe_desc* desc, artlite_mo
   L->shared_gemv_ok = sq && d.hidden % 256 == 0 && d.expert_ffn % 256 == 0 && d.shared_ffn % 256 == 0 &&
                       gemv_supported(sq->id, d.hidden, d.shared_ffn) &&
                       gemv_supported(sdq->id, d.shared_ffn, d.hidden);
+  L->stream_ok = stream_supported(d.gate_type, d.hidden, d.expert_ffn) &&
+                 stream_supported(d.down_type, d.expert_ffn, d.hidden);
+  L->shared_stream_ok = sq && stream_supported(sq->id, d.hidden, d.shared_ffn) &&
+                        stream_supported(sdq->id, d.shared_ffn, d.hidden);
   L->pre_sg = prefill_type(sq);
   L->pre_sd = prefill_type(sdq);
   L->shared_prefill_ok = sq && L->pre_sg && L->pre_sd && prefill_supported(L->pre_sg, d.hidden, d.shared_ffn) &&
