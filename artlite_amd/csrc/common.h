@@ -54,13 +54,36 @@ struct DevBuf {
   ~DevBuf() { release(); }
 };
 
-// A per-thread context of the host-pointer entry points: the current device's stream and scratch buffers.
+// ---- pinned host memory that grows on demand, which kernels read and write in place
+struct PinBuf {
+  void* p = nullptr;
+  size_t n = 0;
+  int reserve(size_t bytes);  // does not keep the contents
+  void release();
+  template <class T>
+  T* as() const { return static_cast<T*>(p); }
+  ~PinBuf() { release(); }
+};
+// The most that a host-pointer call stages each way through its thread's pinned buffers; larger arrays go by pageable
+// copies. (A pageable copy and its synchronization cost 15 to 30 us however small: 16 fp32 tokens of 1024 values through a
+// layer took 129 us with three of them, of which its kernels 51.)
+constexpr size_t PIN_MAX = size_t(4) << 20;
+
+// A per-thread context of the host-pointer entry points: the current device's stream and scratch buffers, and the pinned
+// staging buffers (PIN_MAX each at most; freed with the thread).
 struct HostCtx {
   int device = -1;
   hipStream_t stream = nullptr;
   DevBuf in, out, out2, out3, out4, out5, tmp, tmp2, flag;
+  PinBuf pin_in, pin_out;
 };
 int host_ctx(HostCtx** ctx);
+
+// Copies on the stream by a kernel, between device memory and pinned host memory, whole 4-byte words each: n0 bytes of s0
+// to d0, then (n1 > 0) n1 bytes of s1 to d1, and (zero_words) zeros to that many words of z. A kernel and not a copy
+// engine's transfer, so that the launches around it follow in order with no signal between engines.
+int launch_copy2(void* d0, const void* s0, size_t n0, void* d1, const void* s1, size_t n1, int32_t* z, int zero_words,
+                 hipStream_t s);
 
 // ---- device helpers
 // fp16 bits -> fp32, exact for subnormals (the reference's f16(), csrc/artlite/dequant.cpp:21-29)

@@ -70,6 +70,24 @@ void DevBuf::release() {
   n = 0;
 }
 
+int PinBuf::reserve(size_t bytes) {
+  if (bytes <= n && p) return ARTLITE_OK;
+  release();
+  const size_t want = (bytes + 65536) / 65536 * 65536;
+  void* q = nullptr;
+  hipError_t e = hipHostMalloc(&q, want, hipHostMallocDefault);
+  if (e != hipSuccess) return fail(ARTLITE_ENOMEM, "hipHostMalloc(%zu): %s", want, hipGetErrorString(e));
+  p = q;
+  n = want;
+  return ARTLITE_OK;
+}
+
+void PinBuf::release() {
+  if (p) (void)hipHostFree(p);
+  p = nullptr;
+  n = 0;
+}
+
 namespace {
 struct CtxHolder {
   std::vector<HostCtx*> per_device;
@@ -105,6 +123,44 @@ int host_ctx(HostCtx** out) {
 __global__ void k_copy(const uint4* __restrict__ src, uint4* __restrict__ dst, size_t n) {
   for (size_t i = blockIdx.x * size_t(blockDim.x) + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x)
     dst[i] = src[i];
+}
+
+// 16-byte pieces (all of a thread's loads, which may cross the bus, issued before its first store), then words
+__device__ __forceinline__ void copy_words(uint32_t* d, const uint32_t* s, size_t words) {
+  constexpr int U = 4;
+  const size_t n16 = words / 4, tid = blockIdx.x * size_t(blockDim.x) + threadIdx.x, step = size_t(gridDim.x) * blockDim.x;
+  const uint4* s4 = reinterpret_cast<const uint4*>(s);
+  uint4* d4 = reinterpret_cast<uint4*>(d);
+  for (size_t i = tid; i < n16; i += U * step) {
+    uint4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (i + u * step < n16) v[u] = s4[i + u * step];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (i + u * step < n16) d4[i + u * step] = v[u];
+  }
+  if (tid < words % 4) d[4 * n16 + tid] = s[4 * n16 + tid];
+}
+
+__global__ __launch_bounds__(256) void k_copy2(uint32_t* d0, const uint32_t* s0, size_t w0, uint32_t* d1,
+                                               const uint32_t* s1, size_t w1, int32_t* z, int zw) {
+  copy_words(d0, s0, w0);
+  if (w1) copy_words(d1, s1, w1);
+  if (blockIdx.x == 0 && int(threadIdx.x) < zw) z[threadIdx.x] = 0;
+}
+
+int launch_copy2(void* d0, const void* s0, size_t n0, void* d1, const void* s1, size_t n1, int32_t* z, int zero_words,
+                 hipStream_t s) {
+  const auto bad = [](const void* p, size_t n) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0 || n % 4 != 0; };
+  if (bad(d0, n0) || bad(s0, n0) || (n1 && (bad(d1, n1) || bad(s1, n1))) || zero_words > 256)
+    return fail(ARTLITE_EINVAL, "copy: %zu and %zu bytes, %d words", n0, n1, zero_words);
+  const size_t pieces = n0 / 16 + n1 / 16;
+  const unsigned grid = unsigned(pieces / 512 < 1 ? 1 : pieces / 512 > 256 ? 256 : pieces / 512);
+  k_copy2<<<grid, 256, 0, s>>>(static_cast<uint32_t*>(d0), static_cast<const uint32_t*>(s0), n0 / 4,
+                               static_cast<uint32_t*>(d1), static_cast<const uint32_t*>(s1), n1 / 4, z, zero_words);
+  ART_HIP(hipGetLastError());
+  return ARTLITE_OK;
 }
 
 }  // namespace artlite

@@ -280,6 +280,7 @@ namespace {
 struct PlanMem {
   int32_t *ids, *table, *o2, *o3, *o5, *ctrl;
   int64_t* pos;
+  uint8_t *pin_in = nullptr, *pin_out = nullptr;  // (pinned: the ids; ctrl, o5 and pos; null: pageable copies)
 };
 
 // bytes of each PlanMem region, in order (each followed by a 256-byte tail the vector loads may touch)
@@ -311,38 +312,62 @@ int check_plan_args(const char* who, const int32_t* ids, int64_t n, int k, int E
   return ARTLITE_OK;
 }
 
-// The plan of n x k ids on stream s in the device memory m, the results copied to the caller's host arrays.
+constexpr size_t CTRL_BYTES = (CTRL_WORDS * 4 + 15) / 16 * 16;
+
+// The plan of n x k ids on stream s in the device memory m, the results copied to the caller's host arrays: through pinned
+// memory with one copy each way and one synchronization, or (none) by pageable copies.
 int plan_run(const int32_t* ids, int64_t n, int k, int E, int cols, int cap, int chunk, int32_t* experts,
              int32_t* counts, int32_t* sizes, int32_t* rows, int64_t* pos, const PlanMem& m, hipStream_t s) {
   const int64_t P = n * k;
   const size_t slots = size_t(cols) * cap;
-  if (P) ART_HIP(hipMemcpyAsync(m.ids, ids, size_t(P) * 4, hipMemcpyHostToDevice, s));
-  k_zero_words<<<1, 64, 0, s>>>(m.ctrl, CTRL_WORDS);  // (a fill kernel: no memset node if a caller captures)
-  ART_HIP(hipGetLastError());
+  const size_t o5_bytes = (slots * chunk + 2 * slots + cols) * 4, o5_pad = (o5_bytes + 15) / 16 * 16;
+  if (m.pin_in) {
+    if (P) std::memcpy(m.pin_in, ids, size_t(P) * 4);
+    ART_TRY(launch_copy2(m.ids, m.pin_in, size_t(P) * 4, nullptr, nullptr, 0, m.ctrl, CTRL_WORDS, s));
+  } else {
+    if (P) ART_HIP(hipMemcpyAsync(m.ids, ids, size_t(P) * 4, hipMemcpyHostToDevice, s));
+    k_zero_words<<<1, 64, 0, s>>>(m.ctrl, CTRL_WORDS);  // (a fill kernel: no memset node if a caller captures)
+    ART_HIP(hipGetLastError());
+  }
   DispatchBufs d{m.ids, P, E, k, m.table, m.ctrl, m.o2, m.o2 + E, m.o3, m.o3 + P, nullptr, 0, m.o2 + 2 * E + 1, chunk};
   PlanBufs pl{cols, cap, m.o5 + slots * chunk, m.o5 + slots * chunk + 2 * slots, m.o5 + slots * chunk + slots, m.o5,
               m.pos};
   ART_TRY(launch_plan(d, pl, s));
   int32_t ctrl[CTRL_WORDS];
-  ART_HIP(hipMemcpyAsync(ctrl, m.ctrl, sizeof ctrl, hipMemcpyDeviceToHost, s));
-  ART_HIP(hipStreamSynchronize(s));
+  PlanBufs from = pl;  // (where the results are read)
+  if (m.pin_out) {  // (ctrl and o5, which lie one after the other, then pos)
+    ART_TRY(launch_copy2(m.pin_out, m.ctrl, CTRL_BYTES + o5_bytes, m.pin_out + CTRL_BYTES + o5_pad, m.pos, size_t(P) * 8,
+                         nullptr, 0, s));
+    int32_t* o5 = reinterpret_cast<int32_t*>(m.pin_out + CTRL_BYTES);
+    from = PlanBufs{cols, cap, o5 + slots * chunk, o5 + slots * chunk + 2 * slots, o5 + slots * chunk + slots, o5,
+                    reinterpret_cast<int64_t*>(m.pin_out + CTRL_BYTES + o5_pad)};
+    ART_HIP(hipStreamSynchronize(s));
+    std::memcpy(ctrl, m.pin_out, sizeof ctrl);
+  } else {
+    ART_HIP(hipMemcpyAsync(ctrl, m.ctrl, sizeof ctrl, hipMemcpyDeviceToHost, s));
+    ART_HIP(hipStreamSynchronize(s));
+  }
   if (ctrl[CTRL_BAD]) return fail(ARTLITE_EINVAL, "moe_plan: expert id %d of %d", ids[P - ctrl[CTRL_BAD_FIRST]], E);
   if (ctrl[CTRL_OVER_CAP]) return fail(ARTLITE_EINVAL, "moe_plan: more than %d chunks in a column", cap);
   const int total = ctrl[CTRL_CHUNKS];
-  ART_HIP(hipMemcpyAsync(counts, pl.ccounts, size_t(cols) * 4, hipMemcpyDeviceToHost, s));
+  auto fetch = [&](void* to, const void* at, size_t bytes) -> int {
+    if (m.pin_out)
+      std::memcpy(to, at, bytes);
+    else
+      ART_HIP(hipMemcpyAsync(to, at, bytes, hipMemcpyDeviceToHost, s));
+    return ARTLITE_OK;
+  };
+  ART_TRY(fetch(counts, from.ccounts, size_t(cols) * 4));
   // (only the dealt slots are written: the reference's arrays keep their other entries)
   for (int col = 0; col < cols; col++) {
     const int mc = total > col ? (total - 1 - col) / cols + 1 : 0;
     if (!mc) continue;
-    ART_HIP(hipMemcpyAsync(experts + size_t(col) * cap, pl.experts + size_t(col) * cap, size_t(mc) * 4,
-                           hipMemcpyDeviceToHost, s));
-    ART_HIP(hipMemcpyAsync(sizes + size_t(col) * cap, pl.sizes + size_t(col) * cap, size_t(mc) * 4,
-                           hipMemcpyDeviceToHost, s));
-    ART_HIP(hipMemcpyAsync(rows + size_t(col) * cap * chunk, pl.rows + size_t(col) * cap * chunk,
-                           size_t(mc) * chunk * 4, hipMemcpyDeviceToHost, s));
+    ART_TRY(fetch(experts + size_t(col) * cap, from.experts + size_t(col) * cap, size_t(mc) * 4));
+    ART_TRY(fetch(sizes + size_t(col) * cap, from.sizes + size_t(col) * cap, size_t(mc) * 4));
+    ART_TRY(fetch(rows + size_t(col) * cap * chunk, from.rows + size_t(col) * cap * chunk, size_t(mc) * chunk * 4));
   }
-  if (P) ART_HIP(hipMemcpyAsync(pos, pl.pos, size_t(P) * 8, hipMemcpyDeviceToHost, s));
-  ART_HIP(hipStreamSynchronize(s));
+  if (P) ART_TRY(fetch(pos, from.pos, size_t(P) * 8));
+  if (!m.pin_out) ART_HIP(hipStreamSynchronize(s));
   return ARTLITE_OK;
 }
 
@@ -382,17 +407,23 @@ extern "C" int artlite_moe_plan(const int32_t* ids, int64_t n, int k, int E, int
   ART_TRY(host_ctx(&c));
   size_t b[7];
   plan_sizes(n * k, E, cols, cap, chunk, b);
-  // in: ids | out: table | out2: counts, offsets, cstart | out3: order, slot | out4: pos | out5: rows, experts, sizes,
-  // column counts | flag: ctrl
+  // in: ids | out: table | out2: counts, offsets, cstart | out3: order, slot | out4: pos | out5: ctrl, then rows, experts,
+  // sizes, column counts
   ART_TRY(c->in.reserve(b[0]));
   ART_TRY(c->out.reserve(b[1]));
   ART_TRY(c->out2.reserve(b[2]));
   ART_TRY(c->out3.reserve(b[3]));
   ART_TRY(c->out4.reserve(b[4]));
-  ART_TRY(c->out5.reserve(b[5]));
-  ART_TRY(c->flag.reserve(b[6]));
-  const PlanMem m{c->in.as<int32_t>(), c->out.as<int32_t>(), c->out2.as<int32_t>(), c->out3.as<int32_t>(),
-                  c->out5.as<int32_t>(), c->flag.as<int32_t>(), c->out4.as<int64_t>()};
+  ART_TRY(c->out5.reserve(CTRL_BYTES + b[5]));
+  PlanMem m{c->in.as<int32_t>(), c->out.as<int32_t>(), c->out2.as<int32_t>(), c->out3.as<int32_t>(),
+            c->out5.as<int32_t>() + CTRL_BYTES / 4, c->out5.as<int32_t>(), c->out4.as<int64_t>()};
+  const size_t back = CTRL_BYTES + b[5] + 16 + b[4];
+  if (b[0] <= PIN_MAX && back <= PIN_MAX) {
+    ART_TRY(c->pin_in.reserve(b[0]));
+    ART_TRY(c->pin_out.reserve(back));
+    m.pin_in = c->pin_in.as<uint8_t>();
+    m.pin_out = c->pin_out.as<uint8_t>();
+  }
   return plan_run(ids, n, k, E, cols, cap, chunk, experts, counts, sizes, rows, pos, m, c->stream);
 }
 

@@ -888,11 +888,18 @@ extern "C" int artlite_moe_layer_upload(artlite_moe_layer* L, int t, const void*
   return ARTLITE_OK;
 }
 
-extern "C" int artlite_moe_layer_stage(artlite_moe_layer* L, const void* x, int x_dtype, int64_t T) {
+namespace {
+int check_stage(const artlite_moe_layer* L, const void* x, int x_dtype, int64_t T) {
   if (!L || (!x && T)) return fail(ARTLITE_EINVAL, "moe layer stage: null argument");
   if (T < 0 || T > L->d.max_tokens) return fail(ARTLITE_EINVAL, "moe layer: %lld tokens of at most %d", (long long)T,
                                                 L->d.max_tokens);
   if (x_dtype != ARTLITE_X_F32 && x_dtype != ARTLITE_X_BF16) return fail(ARTLITE_EINVAL, "moe layer: x dtype %d", x_dtype);
+  return ARTLITE_OK;
+}
+}  // namespace
+
+extern "C" int artlite_moe_layer_stage(artlite_moe_layer* L, const void* x, int x_dtype, int64_t T) {
+  ART_TRY(check_stage(L, x, x_dtype, T));
   const size_t bytes = size_t(T) * L->d.hidden * (x_dtype == ARTLITE_X_F32 ? 4 : 2);
   if (bytes) ART_HIP(hipMemcpyAsync(L->x.p, x, bytes, hipMemcpyHostToDevice, L->stream));
   ART_HIP(hipStreamSynchronize(L->stream));
@@ -926,6 +933,29 @@ extern "C" int artlite_moe_layer_output(artlite_moe_layer* L, float* y, int64_t 
 }
 
 extern "C" int artlite_moe_layer_forward(artlite_moe_layer* L, const void* x, int x_dtype, int64_t T, float* y) {
+  ART_TRY(check_stage(L, x, x_dtype, T));
+  const size_t xb = size_t(T) * L->d.hidden * (x_dtype == ARTLITE_X_F32 ? 4 : 2), yb = size_t(T) * L->d.hidden * 4;
+  constexpr size_t CB = (CTRL_WORDS * 4 + 15) / 16 * 16;
+  if (T > 0 && y && xb <= PIN_MAX && CB + yb <= PIN_MAX) {  // (through the thread's pinned buffers: one synchronization)
+    ART_TRY(check_ready(L));
+    HostCtx* c;
+    ART_TRY(host_ctx(&c));
+    ART_TRY(c->pin_in.reserve(xb));
+    ART_TRY(c->pin_out.reserve(CB + yb));
+    std::memcpy(c->pin_in.p, x, xb);
+    ART_TRY(launch_copy2(L->x.p, c->pin_in.p, xb, nullptr, nullptr, 0, nullptr, 0, L->stream));
+    L->x_dtype = x_dtype;
+    L->staged = T;
+    ART_TRY(run(L, T, nullptr));
+    uint8_t* out = c->pin_out.as<uint8_t>();
+    ART_TRY(launch_copy2(out + CB, L->y.p, yb, out, L->ctrl.p, CTRL_WORDS * 4, nullptr, 0, L->stream));
+    ART_HIP(hipStreamSynchronize(L->stream));
+    int32_t ctrl[CTRL_WORDS];
+    std::memcpy(ctrl, out, sizeof ctrl);
+    std::memcpy(y, out + CB, yb);
+    if (ctrl[CTRL_BAD]) return fail(ARTLITE_EHIP, "moe layer: the dispatch saw an invalid expert id");
+    return ARTLITE_OK;
+  }
   ART_TRY(artlite_moe_layer_stage(L, x, x_dtype, T));
   ART_TRY(artlite_moe_layer_run(L, T));
   if (T == 0) {

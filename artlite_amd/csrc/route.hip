@@ -717,6 +717,49 @@ int check_route_args(int64_t n, int per_col, int E, int k) {
 
 using namespace artlite;
 
+namespace {
+// The top k of n tokens' logits from and to host arrays (`need` floats readable at logits, a token's within `ext` of its
+// row; ids n x k, weights w32 or w64). Within PIN_MAX the logits are copied to pinned memory, which the top k reads in
+// place (each logit once) and where it leaves its results: no copies of its own, one synchronization. The tokens go in
+// parts, so that the host's copy of a part runs beside the top k of the one before.
+int route_host(HostCtx* c, const float* logits, size_t need, int64_t n, int64_t row, int64_t ext, int per_col,
+               int64_t pitch, int E, int k, int sigmoid, int32_t* ids, float* w32, double* w64) {
+  const size_t nk = size_t(n) * k, wb = w64 ? 8 : 4;
+  if (need * 4 <= PIN_MAX && nk * (4 + wb) + 16 <= PIN_MAX) {
+    ART_TRY(c->pin_in.reserve(need * 4));
+    ART_TRY(c->pin_out.reserve(nk * (4 + wb) + 16));
+    float* in = c->pin_in.as<float>();
+    uint8_t* wo = c->pin_out.as<uint8_t>();  // (the weights, then the ids)
+    int32_t* io = reinterpret_cast<int32_t*>(wo + nk * wb);
+    // (rows that reach into the next ones: in one part)
+    const int64_t part = row >= ext ? std::max<int64_t>(1, int64_t(1 << 17) / std::max<int64_t>(1, row)) : n;
+    for (int64_t t = 0; t < n; t += part) {
+      const int64_t m = std::min(part, n - t);
+      const size_t at = size_t(t) * size_t(row), end = t + m < n ? size_t(t + m) * size_t(row) : need;
+      std::memcpy(in + at, logits + at, (end - at) * 4);
+      ART_TRY(launch_topk(in + at, m, row, per_col, pitch, E, k, sigmoid, io + t * k,
+                          w64 ? nullptr : reinterpret_cast<float*>(wo) + t * k,
+                          w64 ? reinterpret_cast<double*>(wo) + t * k : nullptr, c->stream));
+    }
+    ART_HIP(hipStreamSynchronize(c->stream));
+    std::memcpy(ids, io, nk * 4);
+    std::memcpy(w64 ? static_cast<void*>(w64) : static_cast<void*>(w32), wo, nk * wb);
+    return ARTLITE_OK;
+  }
+  ART_TRY(c->in.reserve(need * 4));
+  ART_TRY(c->out.reserve(nk * 4));
+  ART_TRY(c->out2.reserve(nk * wb));
+  ART_HIP(hipMemcpyAsync(c->in.p, logits, need * 4, hipMemcpyHostToDevice, c->stream));
+  ART_TRY(launch_topk(c->in.as<float>(), n, row, per_col, pitch, E, k, sigmoid, c->out.as<int32_t>(),
+                      w64 ? nullptr : c->out2.as<float>(), w64 ? c->out2.as<double>() : nullptr, c->stream));
+  ART_HIP(hipMemcpyAsync(ids, c->out.p, nk * 4, hipMemcpyDeviceToHost, c->stream));
+  ART_HIP(hipMemcpyAsync(w64 ? static_cast<void*>(w64) : static_cast<void*>(w32), c->out2.p, nk * wb,
+                         hipMemcpyDeviceToHost, c->stream));
+  ART_HIP(hipStreamSynchronize(c->stream));
+  return ARTLITE_OK;
+}
+}  // namespace
+
 extern "C" int artlite_moe_route(const float* logits, size_t logits_len, int64_t n, int64_t row, int per_col,
                                  int64_t pitch, int E, int k, int sigmoid, int32_t* ids, float* weights) {
   ART_TRY(check_route_args(n, per_col, E, k));
@@ -727,16 +770,8 @@ extern "C" int artlite_moe_route(const float* logits, size_t logits_len, int64_t
   if (int64_t(logits_len) < need) return fail(ARTLITE_EINVAL, "moe_route: arrays too small");
   HostCtx* c;
   ART_TRY(host_ctx(&c));
-  ART_TRY(c->in.reserve(size_t(need) * 4));
-  ART_TRY(c->out.reserve(size_t(n) * k * 4));
-  ART_TRY(c->out2.reserve(size_t(n) * k * 4));
-  ART_HIP(hipMemcpyAsync(c->in.p, logits, size_t(need) * 4, hipMemcpyHostToDevice, c->stream));
-  ART_TRY(launch_topk(c->in.as<float>(), n, row, per_col, pitch, E, k, sigmoid, c->out.as<int32_t>(),
-                      c->out2.as<float>(), nullptr, c->stream));
-  ART_HIP(hipMemcpyAsync(ids, c->out.p, size_t(n) * k * 4, hipMemcpyDeviceToHost, c->stream));
-  ART_HIP(hipMemcpyAsync(weights, c->out2.p, size_t(n) * k * 4, hipMemcpyDeviceToHost, c->stream));
-  ART_HIP(hipStreamSynchronize(c->stream));
-  return ARTLITE_OK;
+  return route_host(c, logits, size_t(need), n, row, int64_t(E / per_col - 1) * pitch + per_col, per_col, pitch, E, k,
+                    sigmoid, ids, weights, nullptr);
 }
 
 extern "C" int artlite_moe_top_k(const float* logits, int64_t n, int E, int k, int sigmoid, int32_t* ids,
@@ -746,14 +781,5 @@ extern "C" int artlite_moe_top_k(const float* logits, int64_t n, int E, int k, i
   if (!logits || !ids || !weights) return fail(ARTLITE_EINVAL, "top_k: null array");
   HostCtx* c;
   ART_TRY(host_ctx(&c));
-  ART_TRY(c->in.reserve(size_t(n) * E * 4));
-  ART_TRY(c->out.reserve(size_t(n) * k * 4));
-  ART_TRY(c->out2.reserve(size_t(n) * k * 8));
-  ART_HIP(hipMemcpyAsync(c->in.p, logits, size_t(n) * E * 4, hipMemcpyHostToDevice, c->stream));
-  ART_TRY(launch_topk(c->in.as<float>(), n, E, E, 0, E, k, sigmoid, c->out.as<int32_t>(), nullptr,
-                      c->out2.as<double>(), c->stream));
-  ART_HIP(hipMemcpyAsync(ids, c->out.p, size_t(n) * k * 4, hipMemcpyDeviceToHost, c->stream));
-  ART_HIP(hipMemcpyAsync(weights, c->out2.p, size_t(n) * k * 8, hipMemcpyDeviceToHost, c->stream));
-  ART_HIP(hipStreamSynchronize(c->stream));
-  return ARTLITE_OK;
+  return route_host(c, logits, size_t(n) * E, n, E, E, E, 0, E, k, sigmoid, ids, nullptr, weights);
 }
