@@ -140,26 +140,40 @@ int check_ready(const artlite_moe_layer* L) {
   return ARTLITE_OK;
 }
 
+// The prefill's routed products by the streamed small tiles (stream.hip): up to STREAM_16 pairs per expert on average in
+// tiles of 16 rows, up to STREAM_32 of 32, then of 64 in the formats that have them (Q4_0, Q4_K, Q8_0; in the others of 32
+// up to STREAM_32_ALONE), up to stream_last pairs: there the MFMA prefill tiles take over. Layer times in us (128 experts
+// 768 wide; 64 rows a tile / 32 / the prefill tiles):
+//   pairs      22               30               35               40               45               50
+//   Q4_0       174 / 170 / 221  190 / 188 / 224  205 / 219 / 228  213 / 242 / 229  250 / 248 / 233  261 / 253 / 234
+//   Q4_K       188 / 178 / 313  218 / 203 / 315  228 / 236 / 302  232 / 254 / 291  283 / 265 / 295  293 / 272 / 291
+//   Q8_0       213 / 220 / 288  238 / 237 / 289  246 / 272 / 290  251 / 298 / 289  275 / 305 / 292  277 / 315 / 294
+// (Q8_0 at 60 pairs 302 / 338 / 296; 32 experts 2880 wide in Q8_0 at 38 / 50 / 58 / 65 pairs 300 / 319 / 339 / 387 in
+// tiles of 64, 366 / 382 / 401 / 464 of 32, 383 / 383 / 385 / 386 on the prefill tiles. Q4_0 at 12.5 / 16 pairs in tiles
+// of 16 138 / 162, of 32 151 / 157.) A shared expert of the routed format joins the prefill tiles' launches and not these
+// (64 experts of Q4_K, 24 / 30 pairs, fp32 x: 259 / 300 against 306 / 294), so the line is lower there.
+constexpr int STREAM_16 = 14, STREAM_32 = 32, STREAM_32_ALONE = 38, STREAM_SHARED = 28;
+constexpr int stream_last(int qtype) { return qtype == ARTLITE_Q8_0 ? 54 : qtype == ARTLITE_Q4_K ? 45 : 41; }
+
+// A shared expert beside streamed routed ones: up to this many tokens on the streamed dense rows, whose launches take its
+// few weight rows 16 tokens at a time, past them on launches of the prefill tiles. (2816 wide, Q4_K, the layer at 64 / 128
+// / 256 / 320 tokens: 166 / 188 / 240 / 276 us against 223 / 235 / 280 / 289, in fp32 175 / 202 / 259 / 300 against 224 /
+// 233 / 281 / 289; 512 wide, Q8_0, 64 / 128 / 180 tokens: 76 / 83 / 87 against 113 / 120 / 123.)
+constexpr int64_t SHARED_STREAM = 256;
+
 // The kernels a forward pass of T tokens takes. Decode-sized passes (at most GEMV_BM pairs per expert on
 // average) run the experts on the VALU GEMV over XQ activations (it takes every block format); larger ones on the
 // fp16 MFMA prefill tiles (every block format: Q4_0, Q8_0, Q4_K from the file's bytes, the others through the prefill
 // layout), and where those do not take a product's shape (K below 320 or not a multiple of 64) on the MFMA decode
 // tiles over bf16 planes. (The GEMV takes widths of partial units in the formats of 32-value blocks: at 8 tokens of 64
 // experts 1408 wide the routed experts took 183 us on the prefill tiles, whose steps are as long for two rows of a tile
-// as for 32, and 47 us on the GEMV; at 5 tokens of 32 experts 2880 wide the layer 215 against 91 us.) (At 128 tokens of config 2, 8 pairs per expert, the prefill tiles' tiles of 32 rows took
-// 208 us against 323 on the MFMA decode tiles: the decode tiles do twice the MFMA work on bf16 hi / lo planes.)
-// The prefill's routed products by the streamed small tiles (stream.hip): up to this many pairs per expert on average in
-// tiles of 16 rows, then of 32, then no longer. Layer times of the 128-expert Q4_0 layer at 200 / 256 / 400 / 512 / 700
-// tokens (12.5 / 16 / 25 / 32 / 44 pairs): tiles of 16 129 / 148 / 196 / 228 / 290 us, of 32 142 / 146 / 161 / 193 /
-// 246 us, the MFMA prefill tiles 208 / 206 / 211 / 215 / 231 us. A shared expert of the routed format joins the prefill
-// tiles' launches and not these (64 experts of Q4_K, 24 / 48 pairs: 268 / 347 against 294 / 302 us), so the line is lower.
-constexpr int STREAM_16 = 14, STREAM_32 = 38, STREAM_32_SHARED = 30;
-
+// as for 32, and 47 us on the GEMV; at 5 tokens of 32 experts 2880 wide the layer 215 against 91 us.) Between
+// them and the prefill sizes the routed products stream (above).
 struct Path {
   bool gemv;            // routed experts (gate / up and down) on the GEMV (XQ of x; tiles of GEMV_BM rows)
   bool shared_gemv;     // the shared expert on the GEMV
   bool prefill;         // routed experts on the prefill tiles
-  int stream;           // ... their products by the streamed small tiles: their rows (16 or 32), 0: not
+  int stream;           // ... their products by the streamed small tiles: their rows (16, 32 or 64), 0: not
   bool shared_prefill;  // the shared expert on the prefill tiles
   bool shared_stream;   // the shared expert on the streamed small tiles (bf16 planes)
   bool split;           // bf16 hi / lo planes of fp32 x needed (the MFMA decode tiles)
@@ -174,15 +188,23 @@ Path path_of(const artlite_moe_layer* L, int64_t T) {
   p.gemv = L->gemv_ok && T * L->d.top_k <= int64_t(GEMV_BM) * L->d.n_experts;
   p.shared_gemv = L->d.shared_ffn && p.gemv && L->shared_gemv_ok;
   p.prefill = !p.gemv && L->prefill_ok;
-  p.shared_prefill = L->d.shared_ffn && p.prefill && L->shared_prefill_ok && T >= 64;
   const int64_t P = T * L->d.top_k, E = L->d.n_experts;
   const bool joins = L->shared_prefill_ok && (L->sq->id == L->gq->id || L->sdq->id == L->dq->id);
-  if (p.prefill && L->stream_ok && P <= int64_t(joins ? STREAM_32_SHARED : STREAM_32) * E) {
-    const int bm = P <= STREAM_16 * E ? 16 : 32;
-    if (stream_fits(L->d.gate_type, true, L->d.expert_ffn, bm, tile_bound(P, int(E), bm)) &&
-        stream_fits(L->d.down_type, false, L->d.hidden, bm, tile_bound(P, int(E), bm)))
+  const int last = joins ? STREAM_SHARED : std::min(stream_last(L->d.gate_type), stream_last(L->d.down_type));
+  if (p.prefill && L->stream_ok && P <= last * E) {
+    const auto fits = [&](int bm) {
+      const int64_t tiles = tile_bound(P, int(E), bm);
+      return stream_fits(L->d.gate_type, true, L->d.expert_ffn, bm, tiles) &&
+             stream_fits(L->d.down_type, false, L->d.hidden, bm, tiles);
+    };
+    const int bm = P <= STREAM_16 * E ? 16 : P <= STREAM_32 * E ? 32 : 64;
+    if (fits(bm))
       p.stream = bm;
+    else if (bm == 64 && P <= STREAM_32_ALONE * E && fits(32))
+      p.stream = 32;
   }
+  p.shared_prefill = L->d.shared_ffn && p.prefill && L->shared_prefill_ok &&
+                     T >= (p.stream && L->shared_stream_ok ? SHARED_STREAM + 1 : 64);
   p.shared_stream = L->d.shared_ffn && !p.shared_gemv && !p.shared_prefill && L->shared_stream_ok;
   const bool planes = (!p.gemv && !p.prefill) || (L->d.shared_ffn && !p.shared_gemv && !p.shared_prefill);
   p.split = planes && (L->x_dtype == ARTLITE_X_F32 || L->d.norm_eps > 0);  // (the normalised x is fp32)

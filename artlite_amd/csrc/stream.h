@@ -1,4 +1,4 @@
-// The streamed small tiles (stream.hip): the experts' grouped products for tiles of at most 32 rows over raw GGUF
+// The streamed small tiles (stream.hip): the experts' grouped products for tiles of at most 64 rows over raw GGUF
 // blocks, on the prefill's fp16 activations, and the same for a few dense rows on bf16 (hi + lo) ones.
 #pragma once
 
@@ -18,7 +18,7 @@ struct StreamArgs {
   const uint16_t* a;        // A's rows of K values
   const int32_t* row_a;     // per sorted row s: its A row (a token); null: A row s
   const float2* row_scale;  // per sorted row
-  int bm;                   // rows of A (tokens for gate / up, pairs for down) of a tile: 16 or 32
+  int bm;                   // rows of A (tokens for gate / up, pairs for down) of a tile: 16, 32 or (Q4_0, Q4_K, Q8_0) 64
   const int32_t* tiles;     // (expert, first sorted row) per tile of bm rows, sorted rows ascending
   const int32_t* n_tiles;   // the tile count (device)
   int64_t max_tiles;        // grid bound

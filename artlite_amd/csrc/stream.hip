@@ -1,4 +1,4 @@
-// The streamed small tiles: the experts' products for tiles of at most 32 rows, on the fp16 or bf16 MFMA (16x16x32) over
+// The streamed small tiles: the experts' products for tiles of at most 64 rows, on the fp16 or bf16 MFMA (16x16x32) over
 // the blocks' integer codes.
 //
 // Numerics. A block's codes are exact in fp16 (1024 + code) and in bf16 (128 + code, codes.h); the activations are the
@@ -14,7 +14,12 @@
 // takes about 22 per row of A and the prefill tiles a step's fixed cost per 64 values of K. The codes are read as aligned
 // dwords: 18-byte blocks read in unaligned pieces took gate / up from 57 to 79 us.
 //
-// Shape of the work. An item is a tile (16 or 32 rows of A at most, one expert's) times 16 WAVES rows of gate and the
+// A tile of 64 rows takes a weight's codes to fp16 and its scale once for up to 64 rows of A, where two tiles of 32 do both
+// again: at 40 rows an expert the Q4_0 layer takes 213 us in tiles of 64, 242 in tiles of 32 and 229 on the prefill tiles
+// (Q4_K: 232, 254, 291; Q8_0: 251, 298, 289). It costs LDS: 4-bit formats then have 1 workgroup of 8 waves a CU.
+//
+// Shape of the work. An item is a tile (16, 32 or 64 rows of A at most, one expert's; its products run over as many
+// 16-row column blocks as it fills) times 16 WAVES rows of gate and the
 // same of up (plain products: 32 WAVES rows); persistent workgroups take items in turn, tile-major. A wave has 2 blocks of
 // 16 weight rows (SwiGLU: gate and up of the same rows, so that h forms in its registers) and streams them, a step of SV
 // values of K at a time, into a ring of LDS slots of its own; the tile's activations for the step, which all waves
@@ -451,6 +456,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((
               n0 = __builtin_amdgcn_readfirstlane(o[3]);
     if (NC == 1 || m <= 16)
       run(std::integral_constant<int, 1>{}, s0, m, n0);
+    else if (NC == 2 || m <= 32)
+      run(std::integral_constant<int, (NC < 2 ? NC : 2)>{}, s0, m, n0);
+    else if (m <= 48)
+      run(std::integral_constant<int, (NC < 3 ? NC : 3)>{}, s0, m, n0);
     else
       run(std::integral_constant<int, NC>{}, s0, m, n0);
   }
@@ -589,11 +598,15 @@ int launch_t(const StreamArgs& a, bool dry, hipStream_t s) {
 }
 
 // (4 waves a workgroup; 8 where the slots then leave one workgroup of 4 a CU: Q6_K's tiles of 32 rows, whose down at 32
-// rows an expert took 110 us with 4 and 93 with 8)
+// rows an expert took 110 us with 4 and 93 with 8. Tiles of 64 rows in the formats they were measured in; Q6_K's slots
+// would not fit them in LDS.)
 template <int QT, int NC>
 int launch_bm(const StreamArgs& a, bool dry, hipStream_t s) {
   constexpr int W = 2 * (SL<QT, true, 4, NC>::LDS + 2048) <= LDS_BYTES ? 4 : 8;
-  return a.w[1] ? launch_t<QT, true, W, NC>(a, dry, s) : launch_t<QT, false, W, NC>(a, dry, s);
+  if constexpr (NC == 4 && QT != ARTLITE_Q4_0 && QT != ARTLITE_Q4_K && QT != ARTLITE_Q8_0)
+    return fail(ARTLITE_EINVAL, "streamed tiles: %d rows of weight type %d", 16 * NC, QT);
+  else
+    return a.w[1] ? launch_t<QT, true, W, NC>(a, dry, s) : launch_t<QT, false, W, NC>(a, dry, s);
 }
 
 }  // namespace
@@ -621,7 +634,9 @@ bool stream_supported(int qtype, int K, int N) {
 namespace {
 int by_type(const StreamArgs& a, bool dry, hipStream_t s) {
 #define ART_ST(QT) \
-  return a.bm == 16 ? launch_bm<QT, 1>(a, dry, s) : launch_bm<QT, 2>(a, dry, s)
+  return a.bm == 16   ? launch_bm<QT, 1>(a, dry, s)  \
+         : a.bm == 32 ? launch_bm<QT, 2>(a, dry, s) \
+                      : launch_bm<QT, 4>(a, dry, s)
   ART_ST_QTYPES(ART_ST)
 #undef ART_ST
 }
@@ -643,7 +658,7 @@ int launch_stream(const StreamArgs& a, hipStream_t s) {
   if (!stream_supported(a.qtype, a.K, a.N))
     return fail(ARTLITE_EINVAL, "streamed tiles: weight type %d, K %d, N %d", a.qtype, a.K, a.N);
   if (!a.w[0] || !a.a || !a.row_scale || (swiglu ? !a.h : !a.y16) || !a.tiles || !a.n_tiles || a.rows < 0 ||
-      (a.bm != 16 && a.bm != 32))
+      (a.bm != 16 && a.bm != 32 && a.bm != 64))
     return fail(ARTLITE_EINVAL, "streamed tiles: null or mismatched argument");
   if (int64_t(a.rows) * a.K * 2 >= (int64_t(1) << 32))
     return fail(ARTLITE_EINVAL, "streamed tiles: %d rows of %d beyond 32-bit offsets", a.rows, a.K);

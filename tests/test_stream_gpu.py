@@ -1,6 +1,9 @@
 """The streamed small tiles (past the GEMV's sizes, up to a few dozen pairs per expert) against float64 math, in every
-block format: token counts around the line between tiles of 16 and of 32 rows and the first and last that take them,
-widths of partial K-units and of partial 64-row blocks, tiles of one row and of a full one (uneven routing)."""
+block format: token counts around the lines between tiles of 16, 32 and 64 rows and the first and last that take them,
+widths of partial K-units and of partial 64-row blocks, tiles of one row and of a full one (uneven routing); a shared expert
+beside them on either side of its own line."""
+
+from dataclasses import replace
 
 import numpy as np
 import pytest
@@ -25,16 +28,30 @@ CASES = [
     Spec("iq4_xs", H=512, E=8, k=2, F=512, gate_type="IQ4_XS", down_type="Q4_K", scale=5e-5, dmin_scale=1.5e-3),
 ]
 TOKENS = (17, 56, 57, 152)
+# (the formats with tiles of 64 rows: from 33 pairs per expert, up to 41, 45 and 54; then the first of the prefill tiles)
+LAST = {"q4_0": 41, "q8_0": 41, "q4_k": 45, "q8_0_only": 54}
+CASES_64 = [
+    CASES[0], CASES[1],
+    Spec("q4_k", H=512, E=8, k=2, F=512, gate_type="Q4_K", down_type="Q8_0", scale=2e-4, dmin_scale=1.5e-3),
+    Spec("q8_0_only", H=448, E=8, k=2, F=576, gate_type="Q8_0", down_type="Q8_0", scale=0.01),
+]
+# (a shared expert beside streamed routed ones: on the streamed dense rows up to 256 tokens, then on the prefill tiles; 16
+# experts, whose few logits leave no near tie among 63 to 65 tokens, where one is more than the oracle's check allows)
+SHARED = Spec("shared", H=512, E=16, k=2, F=384, gate_type="Q4_0", down_type="Q8_0", scale=0.02, shared_F=448,
+              shared_type="Q8_0", shared_down_type="Q4_0", shared_gated=True)
 
 
-@pytest.mark.parametrize("spec", CASES, ids=[s.name for s in CASES])
-def test_stream_tiles(spec: Spec) -> None:
+@pytest.mark.parametrize(("spec", "tokens"),
+                         [(s, TOKENS) for s in CASES]
+                         + [(s, (132, 133, LAST[s.name] * 4, LAST[s.name] * 4 + 1)) for s in CASES_64]
+                         + [(replace(SHARED, x_dtype=x), (63, 64, 65, 256, 257)) for x in ("bf16", "f32")])
+def test_stream_tiles(spec: Spec, tokens: tuple) -> None:
     layer = layers.make_layer(spec, 7)
     # (uneven: expert 0 far ahead, expert 1 behind, so that tiles of every size come up)
     layer.router[0] += 0.08
     layer.router[1] -= 0.08
-    with gpu_layer(layer, max_tokens=max(TOKENS)) as g:
-        for T in TOKENS + TOKENS[:1]:
+    with gpu_layer(layer, max_tokens=max(tokens)) as g:
+        for T in tokens + tokens[:1]:
             x = np.abs(layers.make_x(spec, T, T))
             y = g(gpu_input(spec, x))
             names = g.kernel_names()
