@@ -15,7 +15,7 @@ CSRC = PKG / "csrc"
 OUT = PKG / "libartlite_moe.so"
 ARCH = "gfx950"
 
-# all device code: gfx950 only; packed fp32 instructions off (they are not trusted on the target pool)
+# all device code: gfx950 only; packed fp32 instructions off (some of their forms are not trusted on the target)
 COMMON = ["-std=c++17", "-O3", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
           "-packed-fp32-ops", "-Wall", "-Wno-unused-result"]
 # per-file extra flags: the dequantizer's fp32 operations in the reference's order, unfused; the prefill tiles with the
