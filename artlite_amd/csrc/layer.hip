@@ -715,8 +715,6 @@ extern "C" int artlite_moe_layer_create(const artlite_moe_desc* desc, artlite_mo
     L->sgate_row = size_t(d.hidden) / sq->per * sq->dev;
     L->sdown_row = size_t(d.shared_ffn) / sdq->per * sdq->dev;
   }
-  L->gemv_ok = gemv_supported(d.gate_type, d.hidden, d.expert_ffn) &&
-               gemv_supported(d.down_type, d.expert_ffn, d.hidden);
   // (the prefill tiles address weights and A rows by 32-bit offsets: every expert's bytes, every row of x16 and h16)
   const int64_t maxP = int64_t(d.max_tokens) * d.top_k;
   L->pre_g = prefill_type(gq);
@@ -727,6 +725,12 @@ extern "C" int artlite_moe_layer_create(const artlite_moe_desc* desc, artlite_mo
                                d.max_tokens, d.hidden) &&
                   prefill_fits(d.n_experts, int64_t(d.hidden) * prefill_row(L->down_row, d.expert_ffn, L->pre_d), maxP,
                                d.expert_ffn);
+  // (widths of partial units take the GEMV in place of the prefill tiles' fp16 products. Layers that have none, widths of
+  // 64, 128 and 192 among them, keep the MFMA decode tiles, whose bf16 hi / lo planes hold x and h to 2^-17 where XQ
+  // holds them to 2^-16 of a group's largest: 192 wide 3.7e-6 to 5e-6 against 64 bits, on the GEMV 4.3e-5 to 4.6e-5.)
+  L->gemv_ok = gemv_supported(d.gate_type, d.hidden, d.expert_ffn) &&
+               gemv_supported(d.down_type, d.expert_ffn, d.hidden) &&
+               ((d.hidden % 256 == 0 && d.expert_ffn % 256 == 0) || L->prefill_ok);
   // (a shared expert beside routed ones of a partial unit stays on the MFMA decode tiles: its bf16 hi / lo planes hold
   // x and h to 2^-17, XQ to 2^-16 of a group's largest, and its output is the layer's largest term)
   L->shared_gemv_ok = sq && d.hidden % 256 == 0 && d.expert_ffn % 256 == 0 && d.shared_ffn % 256 == 0 &&

@@ -1,0 +1,20 @@
+"""Which kernels a pass takes, on the CPU: the names of a layer's kernels by format, widths and token count."""
+
+from pathlib import Path
+
+import pytest
+
+from .fake_runtime import run_fake
+
+
+@pytest.mark.parametrize(("H", "F", "fmt", "gemv"), [(2048, 192, "Q4_0", False), (64, 1408, "Q8_0", False),
+                                                     (128, 128, "Q4_1", False), (192, 512, "IQ4_NL", False),
+                                                     (2048, 320, "Q4_0", True), (2880, 2880, "Q8_0", True),
+                                                     (256, 256, "Q4_0", True), (512, 256, "Q4_K", True)])
+def test_decode_widths(tmp_path: Path, H: int, F: int, fmt: str, gemv: bool) -> None:
+    """Decode of widths of partial units is the GEMV's where the prefill tiles take them, and stays on the MFMA decode
+    tiles' bf16 planes below that; whole units of 256 are the GEMV's at any width."""
+    run_fake(tmp_path, f"""
+n = names(8, hidden={H}, n_experts=16, top_k=4, expert_ffn={F}, gate_type="{fmt}", down_type="{fmt}")
+assert ("router_quant" in n) == {gemv} and "prefill_x" not in n, n
+""")
