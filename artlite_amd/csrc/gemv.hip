@@ -582,12 +582,26 @@ __device__ __forceinline__ float row4_sum(float s) {
   return __uint_as_float(y[0]) + __uint_as_float(y[1]);
 }
 
+// Whole units or partial ones (P): of K (a row's last unit is partly past its end), or of N alone (SwiGLU: so are the XQ rows
+// of h that it writes). The counts of units are K / 256 and N / 256 in the kernels of whole ones, which compile as if there
+// were no others: (K + 255) / 256 for all took Q4_0's gate / up from 16 to 19 spilled SGPRs and its down from 84 to 98
+// SGPRs, and 16 tokens of 128 experts 768 wide from 78.2 to 78.6 us.
+constexpr int WHOLE = 0, PART_N = 1, PART_K = 2;
+template <int P>
+__device__ __forceinline__ int k_units(int K) {
+  return P == PART_K ? xq_units(K) : K / 256;
+}
+template <int P>
+__device__ __forceinline__ int n_units(int N) {
+  return P == WHOLE ? N / 256 : xq_units(N);
+}
+
 // The state of a wave's stream of steps over its items (one step: 16 rows x one K-unit of one matrix). Every load
 // of the stream is a DMA into LDS (the weights into D slots, the records of a K-unit into one slot), counted as it
 // is issued (nl), so that each wait names the exact number of loads issued after the ones it needs: loads of one kind
 // return in order. (Records loaded into registers instead would make the compiler wait for all loads in flight
 // before each use: it cannot order them against the DMAs.)
-template <int QT, bool SWIGLU, int D>
+template <int QT, bool SWIGLU, int D, int P>
 struct Stream {
   using W = Shape<SWIGLU>;
   static constexpr int RB = W::RB, S = W::S, BY = Unit<QT>::BYTES, CH = BY / 16, LW = Unit<QT>::LW;
@@ -611,7 +625,7 @@ struct Stream {
     lane = threadIdx.x & 63, p = lane >> 4, r = lane & 15;
     rb = wv / S, ks = wv % S;
     my = slab + wv * (D * WCH + XCH);
-    const int U = xq_units(a.K);
+    const int U = k_units<P>(a.K);
     u0 = ks;  // (the wave's K-units: ks, ks + S, ...; the pair reads neighbouring units, which share lines, together)
     NVw = (U - ks + S - 1) / S * NM;
 #pragma unroll
@@ -663,7 +677,7 @@ struct Stream {
     for (int t = 0; t < GEMV_BM; t++)
       if (t < I.m)
         __builtin_amdgcn_global_load_lds(
-            reinterpret_cast<const void*>(a.xq + int64_t(I.ar[t]) * xq_row_dwords(a.K) + ku * XQ_UNIT + 4 * lane),
+            reinterpret_cast<const void*>(a.xq + int64_t(I.ar[t]) * (int64_t(k_units<P>(a.K)) * XQ_UNIT) + ku * XQ_UNIT + 4 * lane),
             (__attribute__((address_space(3))) void*)(dst + 64 * t), 16, 0, 0);
     nl += I.m;
     xend = nl;
@@ -673,10 +687,10 @@ struct Stream {
 // the wait and read of a step: vmcnt(n), then the weights and (MX) the record chunks. n is at most NMAX (the stream's
 // counts: after a step's weights come the LA steps' issued ahead (NI each) and at most LA + 1 K-units' records); a
 // larger n, which the stream does not produce, would wait for every load (vmcnt(0)), never for fewer than needed
-template <int QT, bool SWIGLU, int MX, int D>
-__device__ __forceinline__ void wait_read(const Stream<QT, SWIGLU, D>& st, int n, uint32_t sw, uint32_t sx,
+template <int QT, bool SWIGLU, int MX, int D, int P>
+__device__ __forceinline__ void wait_read(const Stream<QT, SWIGLU, D, P>& st, int n, uint32_t sw, uint32_t sx,
                                           uint32_t (&w)[Unit<QT>::LW], u32x4 (&x)[GEMV_BM]) {
-  using SS = Stream<QT, SWIGLU, D>;
+  using SS = Stream<QT, SWIGLU, D, P>;
   if (n > SS::NMAX) n = 0;
   static_for<SS::NMAX + 1>([&](auto nc) {
     constexpr int N = decltype(nc)::value;
@@ -685,10 +699,10 @@ __device__ __forceinline__ void wait_read(const Stream<QT, SWIGLU, D>& st, int n
   read_unit<QT, MX>(w, x, sw + st.o_w, sw + st.o_r, sw + st.o_s, sx);
 }
 
-// The dot products of one step: the lane's two groups of the unit w against the M rows of A's records x. RAG: a row's
-// last unit may be partly past its end; !on: the lane's groups are (its scales, then bytes of whatever follows the
+// The dot products of one step: the lane's two groups of the unit w against the M rows of A's records x. PART_K: a
+// row's last unit may be partly past its end; !on: the lane's groups are (its scales, then bytes of whatever follows the
 // row, taken as 0, as the records' are).
-template <int QT, int M, bool RAG>
+template <int QT, int M, int P>
 __device__ __forceinline__ void step_terms(const uint32_t (&w)[Unit<QT>::LW], const u32x4 (&x)[GEMV_BM], int p, bool on,
                                            float (&acc)[M]) {
   static_for<2>([&](auto hc) {
@@ -696,7 +710,7 @@ __device__ __forceinline__ void step_terms(const uint32_t (&w)[Unit<QT>::LW], co
     uint32_t q[8];
     float d, mn;
     codes<QT, H>(w, 2 * p + H, q, d, mn);
-    if constexpr (RAG) d = on ? d : 0.0f, mn = on ? mn : 0.0f;
+    if constexpr (P == PART_K) d = on ? d : 0.0f, mn = on ? mn : 0.0f;
 #pragma unroll
     for (int t = 0; t < M; t++) acc[t] = group_term<QT, H>(acc[t], x[t][H], x[t][2], x[t][3], q, d, mn);
   });
@@ -707,10 +721,10 @@ __device__ __forceinline__ void step_terms(const uint32_t (&w)[Unit<QT>::LW], co
 // the weights LA steps ahead, then waits for its own; at the start of each K-unit that wait also covers the
 // records, which are read into registers with the weights, and the next K-unit's are loaded into the freed slot.
 // Returns with the sums of the four lanes of a row in every lane.
-template <int QT, bool SWIGLU, int M, int D, bool RAG>
-__device__ __forceinline__ void run_item(Stream<QT, SWIGLU, D>& st, const Item& cur, const Item& nxt, bool has_next,
+template <int QT, bool SWIGLU, int M, int D, int P>
+__device__ __forceinline__ void run_item(Stream<QT, SWIGLU, D, P>& st, const Item& cur, const Item& nxt, bool has_next,
                                          int gs, float (&out)[SWIGLU ? 2 : 1][GEMV_BM]) {
-  using SS = Stream<QT, SWIGLU, D>;
+  using SS = Stream<QT, SWIGLU, D, P>;
   constexpr int NM = SS::NM, LW = SS::LW, LA = SS::LA;
   float acc[NM][M];
 #pragma unroll
@@ -718,9 +732,9 @@ __device__ __forceinline__ void run_item(Stream<QT, SWIGLU, D>& st, const Item& 
 #pragma unroll
     for (int t = 0; t < M; t++) acc[mx][t] = 0.0f;
   u32x4 xc[GEMV_BM];
-  const int pv = RAG ? (st.a.K % 256) / 64 : 0;  // (RAG: the lane rows p < pv hold groups of the last unit)
+  const int pv = P == PART_K ? (st.a.K % 256) / 64 : 0;  // (the lane rows p < pv hold groups of the last unit)
   for (int v0 = 0; v0 < st.NVw; v0 += NM) {
-    const bool on = !RAG || st.p < pv || st.u0 + SS::S * (v0 / NM) < st.a.K / 256;
+    const bool on = P != PART_K || st.p < pv || st.u0 + SS::S * (v0 / NM) < st.a.K / 256;
     static_for<NM>([&](auto jc) {
       constexpr int MX = decltype(jc)::value;
       const int v = v0 + MX;
@@ -737,15 +751,15 @@ __device__ __forceinline__ void run_item(Stream<QT, SWIGLU, D>& st, const Item& 
       if constexpr (MX == 0) {
         // (wend[D - 1]: this step's weights), then the next K-unit's records into the slot just read
         const int nw = st.nl - st.wend[D - 1];
-        wait_read<QT, SWIGLU, M, D>(st, min(nw, st.nl - st.xend), sw, st.xbase, w, xc);
+        wait_read<QT, SWIGLU, M, D, P>(st, min(nw, st.nl - st.xend), sw, st.xbase, w, xc);
         if (v0 + NM < st.NVw)
           st.load_x(cur, st.u0 + SS::S * (v0 / NM + 1));
         else if (has_next)
           st.load_x(nxt, st.u0);
       } else {
-        wait_read<QT, SWIGLU, 0, D>(st, st.nl - st.wend[D - 1], sw, st.xbase, w, xc);
+        wait_read<QT, SWIGLU, 0, D, P>(st, st.nl - st.wend[D - 1], sw, st.xbase, w, xc);
       }
-      step_terms<QT, M, RAG>(w, xc, st.p, on, acc[MX]);
+      step_terms<QT, M, P>(w, xc, st.p, on, acc[MX]);
     });
   }
 #pragma unroll
@@ -761,11 +775,11 @@ __device__ __forceinline__ void run_item(Stream<QT, SWIGLU, D>& st, const Item& 
 }
 
 // A persistent workgroup: items snake_item(blockIdx.x, j, gridDim.x) of (tile, block of 16 RB rows), tile-major.
-template <int QT, bool SWIGLU, int D, bool RAG>
+template <int QT, bool SWIGLU, int D, int P>
 __global__ __launch_bounds__(Shape<SWIGLU>::THREADS) __attribute__((amdgpu_waves_per_eu(QT == ARTLITE_Q4_0 ? 4 : 2))) void k_gemv(
     const GemvArgs a) {
   using W = Shape<SWIGLU>;
-  using SS = Stream<QT, SWIGLU, D>;
+  using SS = Stream<QT, SWIGLU, D, P>;
   constexpr int RB = W::RB, S = W::S, NM = SS::NM;
   const int rows = 16 * RB, NB = (a.N + rows - 1) / rows;
   extern __shared__ u32x4 slab[];
@@ -847,10 +861,10 @@ __global__ __launch_bounds__(Shape<SWIGLU>::THREADS) __attribute__((amdgpu_waves
     if (has_next) nxt = get_item(tab, j + 1);
     float out[NM][GEMV_BM];
     switch (cur.m) {
-      case 1: run_item<QT, SWIGLU, 1, D, RAG>(st, cur, nxt, has_next, gs, out); break;
-      case 2: run_item<QT, SWIGLU, 2, D, RAG>(st, cur, nxt, has_next, gs, out); break;
-      case 3: run_item<QT, SWIGLU, 3, D, RAG>(st, cur, nxt, has_next, gs, out); break;
-      default: run_item<QT, SWIGLU, 4, D, RAG>(st, cur, nxt, has_next, gs, out); break;
+      case 1: run_item<QT, SWIGLU, 1, D, P>(st, cur, nxt, has_next, gs, out); break;
+      case 2: run_item<QT, SWIGLU, 2, D, P>(st, cur, nxt, has_next, gs, out); break;
+      case 3: run_item<QT, SWIGLU, 3, D, P>(st, cur, nxt, has_next, gs, out); break;
+      default: run_item<QT, SWIGLU, 4, D, P>(st, cur, nxt, has_next, gs, out); break;
     }
     gs += st.NVw;
     if constexpr (!SWIGLU) {
@@ -882,7 +896,7 @@ __global__ __launch_bounds__(Shape<SWIGLU>::THREADS) __attribute__((amdgpu_waves
           // lanes 8 RB / 2 t .. + 8 RB / 2 take row of A t: 8 lanes per XQ group of 32 rows, 4 rows each
           constexpr int LPT = 8 * RB / 2;
           const int t = ln / LPT, lt = ln % LPT, l8 = lt & 7, rbb = lt >> 2, r0 = 4 * (lt & 3);
-          const int UH = xq_units(a.N), blk = cur.n0 / 32 + (lt >> 3), g = blk & 7;
+          const int UH = n_units<P>(a.N), blk = cur.n0 / 32 + (lt >> 3), g = blk & 7;
           float4 gsum = {0.0f, 0.0f, 0.0f, 0.0f}, usum = gsum;
 #pragma unroll
           for (int k = 0; k < S; k++) {
@@ -926,14 +940,14 @@ int64_t gemv_items(const GemvArgs& a) {
   return tiles * ((a.N + 16 * W::RB - 1) / (16 * W::RB));
 }
 
-// persistent workgroups of k_gemv<QT, SWIGLU, D, RAG>: as many as the device holds at once (queried once per kernel, with
+// persistent workgroups of k_gemv<QT, SWIGLU, D, P>: as many as the device holds at once (queried once per kernel, with
 // a table of 64 items; 0: set-up failed); their item tables take 32 bytes an item, at most lds_max in all
-template <int QT, bool SWIGLU, int D, bool RAG>
+template <int QT, bool SWIGLU, int D, int P>
 int gemv_resident() {
   using W = Shape<SWIGLU>;
   constexpr size_t lds0 = gemv_lds<QT, SWIGLU, D>(), lds_max = lds0 + 8192;
   static const int resident = [] {
-    const void* f = reinterpret_cast<const void*>(k_gemv<QT, SWIGLU, D, RAG>);
+    const void* f = reinterpret_cast<const void*>(k_gemv<QT, SWIGLU, D, P>);
     int dev = 0, cus = 0, per_cu = 0;
     if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds_max)) != hipSuccess ||
         hipGetDevice(&dev) != hipSuccess ||
@@ -945,14 +959,14 @@ int gemv_resident() {
   return resident;
 }
 
-template <int QT, bool SWIGLU, int D, bool RAG>
+template <int QT, bool SWIGLU, int D, int P>
 int launch_t(const GemvArgs& a, hipStream_t s) {
   using W = Shape<SWIGLU>;
   const int64_t items = gemv_items<SWIGLU>(a);
   if (items <= 0) return ARTLITE_OK;
   if (items >= (int64_t(1) << 31)) return fail(ARTLITE_EINVAL, "expert GEMV: %lld work items", (long long)items);
   constexpr size_t lds0 = gemv_lds<QT, SWIGLU, D>(), lds_max = lds0 + 8192;
-  const int resident = gemv_resident<QT, SWIGLU, D, RAG>();
+  const int resident = gemv_resident<QT, SWIGLU, D, P>();
   if (resident <= 0) return fail(ARTLITE_EHIP, "expert GEMV: kernel set-up failed");
   const unsigned grid = unsigned(std::min<int64_t>(items, resident));
   const size_t lds = lds0 + size_t((items + grid - 1) / grid) * 32;
@@ -968,7 +982,7 @@ int launch_t(const GemvArgs& a, hipStream_t s) {
       return fail(ARTLITE_EINVAL, "expert GEMV: routing of %d tokens, %d experts, top %d in the launch", r.T, r.E,
                   r.k);
   }
-  k_gemv<QT, SWIGLU, D, RAG><<<grid, W::THREADS, lds, s>>>(a);
+  k_gemv<QT, SWIGLU, D, P><<<grid, W::THREADS, lds, s>>>(a);
   ART_HIP(hipGetLastError());
   return ARTLITE_OK;
 }
@@ -1005,13 +1019,14 @@ int launch_gemv(const GemvArgs& a, hipStream_t s) {
   const bool swiglu = a.w[1] != nullptr;
   if (swiglu && !a.hq) return fail(ARTLITE_EINVAL, "expert GEMV: no h");
   if (!swiglu && !a.y) return fail(ARTLITE_EINVAL, "expert GEMV: no output");
-  // (a K of partial units: kernels of their own for the formats that have them, so that the others' steps are as
-  // they were)
+  // (partial units of K, which only the formats of 32-value blocks have, and of a SwiGLU product's N: kernels of their own)
+  const bool part_n = swiglu && a.N % 256;
 #define ART_DISPATCH(QT)                                                                                   \
-  return swiglu ? launch_t<QT, true, WSLOTS, false>(a, s) : launch_t<QT, false, WSLOTS, false>(a, s)
+  if (part_n) return launch_t<QT, true, WSLOTS, PART_N>(a, s);                                             \
+  return swiglu ? launch_t<QT, true, WSLOTS, WHOLE>(a, s) : launch_t<QT, false, WSLOTS, WHOLE>(a, s)
 #define ART_DISPATCH_32(QT)                                                                                \
   if (a.K % 256)                                                                                           \
-    return swiglu ? launch_t<QT, true, WSLOTS, true>(a, s) : launch_t<QT, false, WSLOTS, true>(a, s);      \
+    return swiglu ? launch_t<QT, true, WSLOTS, PART_K>(a, s) : launch_t<QT, false, WSLOTS, PART_K>(a, s);  \
   ART_DISPATCH(QT)
   switch (a.qtype) {
     case ARTLITE_Q4_0: ART_DISPATCH_32(ARTLITE_Q4_0);
