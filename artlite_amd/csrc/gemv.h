@@ -62,6 +62,9 @@ bool gemv_route_fits(int64_t T, int E, int k);
 // 32-value blocks) a multiple of 64, whose last unit is partly past the row's end; N whole items of 64 rows
 bool gemv_supported(int qtype, int K, int N);
 
+// whether a launch of these takes every item of max_tiles tiles (its workgroups' item tables, 256 items each at most)
+bool gemv_fits(int qtype, bool swiglu, int K, int N, int64_t max_tiles);
+
 int launch_gemv(const GemvArgs& a, hipStream_t s);
 
 // one XQ row back to fp32 (host side, for inspection)

@@ -960,17 +960,18 @@ int gemv_resident() {
 }
 
 template <int QT, bool SWIGLU, int D, int P>
-int launch_t(const GemvArgs& a, hipStream_t s) {
+int launch_t(const GemvArgs& a, bool dry, hipStream_t s) {
   using W = Shape<SWIGLU>;
   const int64_t items = gemv_items<SWIGLU>(a);
   if (items <= 0) return ARTLITE_OK;
-  if (items >= (int64_t(1) << 31)) return fail(ARTLITE_EINVAL, "expert GEMV: %lld work items", (long long)items);
   constexpr size_t lds0 = gemv_lds<QT, SWIGLU, D>(), lds_max = lds0 + 8192;
   const int resident = gemv_resident<QT, SWIGLU, D, P>();
   if (resident <= 0) return fail(ARTLITE_EHIP, "expert GEMV: kernel set-up failed");
   const unsigned grid = unsigned(std::min<int64_t>(items, resident));
   const size_t lds = lds0 + size_t((items + grid - 1) / grid) * 32;
-  if (lds > lds_max) return fail(ARTLITE_EINVAL, "expert GEMV: %lld work items", (long long)items);
+  const bool fits = items < (int64_t(1) << 31) && lds <= lds_max;
+  if (dry) return fits ? ARTLITE_OK : ARTLITE_EINVAL;
+  if (!fits) return fail(ARTLITE_EINVAL, "expert GEMV: %lld work items", (long long)items);
   if (SWIGLU && a.route.logits) {
     // the routing's LDS (scratch, then the tile list, order, offsets and tile count) within the slots
     const GemvArgs::Route& r = a.route;
@@ -1009,24 +1010,17 @@ bool gemv_supported(int qtype, int K, int N) {
   return (gemv_blocks32(qtype) || k256) && K > 0 && K % (k256 ? 256 : 64) == 0 && N > 0 && N % 64 == 0;
 }
 
-int launch_gemv(const GemvArgs& a, hipStream_t s) {
-  if (!gemv_supported(a.qtype, a.K, a.N))
-    return fail(ARTLITE_EINVAL,
-                "expert GEMV: weight type %d with K %d, N %d (K a multiple of 256, or of 64 in 32-value blocks, N of 64)",
-                a.qtype, a.K, a.N);
-  if (a.N <= 0 || int64_t(a.N) * a.row_bytes >= (int64_t(1) << 31))
-    return fail(ARTLITE_EINVAL, "expert GEMV: %d rows of %d bytes", a.N, a.row_bytes);
-  const bool swiglu = a.w[1] != nullptr;
-  if (swiglu && !a.hq) return fail(ARTLITE_EINVAL, "expert GEMV: no h");
-  if (!swiglu && !a.y) return fail(ARTLITE_EINVAL, "expert GEMV: no output");
+namespace {
+// (dry: whether a launch takes the items, as a status and no message)
+int by_type(const GemvArgs& a, bool dry, hipStream_t s) {
   // (partial units of K, which only the formats of 32-value blocks have, and of a SwiGLU product's N: kernels of their own)
-  const bool part_n = swiglu && a.N % 256;
+  const bool swiglu = a.w[1] != nullptr, part_n = swiglu && a.N % 256;
 #define ART_DISPATCH(QT)                                                                                   \
-  if (part_n) return launch_t<QT, true, WSLOTS, PART_N>(a, s);                                             \
-  return swiglu ? launch_t<QT, true, WSLOTS, WHOLE>(a, s) : launch_t<QT, false, WSLOTS, WHOLE>(a, s)
+  if (part_n) return launch_t<QT, true, WSLOTS, PART_N>(a, dry, s);                                             \
+  return swiglu ? launch_t<QT, true, WSLOTS, WHOLE>(a, dry, s) : launch_t<QT, false, WSLOTS, WHOLE>(a, dry, s)
 #define ART_DISPATCH_32(QT)                                                                                \
   if (a.K % 256)                                                                                           \
-    return swiglu ? launch_t<QT, true, WSLOTS, PART_K>(a, s) : launch_t<QT, false, WSLOTS, PART_K>(a, s);  \
+    return swiglu ? launch_t<QT, true, WSLOTS, PART_K>(a, dry, s) : launch_t<QT, false, WSLOTS, PART_K>(a, dry, s);  \
   ART_DISPATCH(QT)
   switch (a.qtype) {
     case ARTLITE_Q4_0: ART_DISPATCH_32(ARTLITE_Q4_0);
@@ -1041,6 +1035,30 @@ int launch_gemv(const GemvArgs& a, hipStream_t s) {
   }
 #undef ART_DISPATCH_32
 #undef ART_DISPATCH
+}
+}  // namespace
+
+bool gemv_fits(int qtype, bool swiglu, int K, int N, int64_t max_tiles) {
+  static const uint8_t up = 0;
+  static const int32_t list = 0;
+  GemvArgs a{};
+  a.w[1] = swiglu ? &up : nullptr;  // (the kinds alone)
+  a.tiles = &list;
+  a.qtype = qtype, a.K = K, a.N = N, a.max_tiles = max_tiles;
+  return by_type(a, true, nullptr) == ARTLITE_OK;
+}
+
+int launch_gemv(const GemvArgs& a, hipStream_t s) {
+  if (!gemv_supported(a.qtype, a.K, a.N))
+    return fail(ARTLITE_EINVAL,
+                "expert GEMV: weight type %d with K %d, N %d (K a multiple of 256, or of 64 in 32-value blocks, N of 64)",
+                a.qtype, a.K, a.N);
+  if (a.N <= 0 || int64_t(a.N) * a.row_bytes >= (int64_t(1) << 31))
+    return fail(ARTLITE_EINVAL, "expert GEMV: %d rows of %d bytes", a.N, a.row_bytes);
+  const bool swiglu = a.w[1] != nullptr;
+  if (swiglu && !a.hq) return fail(ARTLITE_EINVAL, "expert GEMV: no h");
+  if (!swiglu && !a.y) return fail(ARTLITE_EINVAL, "expert GEMV: no output");
+  return by_type(a, false, s);
 }
 
 void xq_dequant_row(const uint32_t* row, int K, float* out) {

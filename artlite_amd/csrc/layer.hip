@@ -185,10 +185,14 @@ struct Path {
 
 Path path_of(const artlite_moe_layer* L, int64_t T) {
   Path p{};
-  p.gemv = L->gemv_ok && T * L->d.top_k <= int64_t(GEMV_BM) * L->d.n_experts;
+  const int64_t P = T * L->d.top_k, E = L->d.n_experts;
+  if (L->gemv_ok && P <= GEMV_BM * E) {  // (about a thousand experts 3000 to 4000 wide have more tiles than its launches take)
+    const int64_t tiles = tile_bound(P, int(E), GEMV_BM);
+    p.gemv = gemv_fits(L->d.gate_type, true, L->d.hidden, L->d.expert_ffn, tiles) &&
+             gemv_fits(L->d.down_type, false, L->d.expert_ffn, L->d.hidden, tiles);
+  }
   p.shared_gemv = L->d.shared_ffn && p.gemv && L->shared_gemv_ok;
   p.prefill = !p.gemv && L->prefill_ok;
-  const int64_t P = T * L->d.top_k, E = L->d.n_experts;
   const bool joins = L->shared_prefill_ok && (L->sq->id == L->gq->id || L->sdq->id == L->dq->id);
   const int last = joins ? STREAM_SHARED : std::min(stream_last(L->d.gate_type), stream_last(L->d.down_type));
   if (p.prefill && L->stream_ok && P <= last * E) {

@@ -18,3 +18,17 @@ def test_decode_widths(tmp_path: Path, H: int, F: int, fmt: str, gemv: bool) -> 
 n = names(8, hidden={H}, n_experts=16, top_k=4, expert_ffn={F}, gate_type="{fmt}", down_type="{fmt}")
 assert ("router_quant" in n) == {gemv} and "prefill_x" not in n, n
 """)
+
+
+@pytest.mark.parametrize(("H", "F"), [(1280, 2944), (320, 4032)])
+def test_decode_of_many_wide_experts(tmp_path: Path, H: int, F: int) -> None:
+    """1024 experts at 4 pairs each, more items than the GEMV's workgroups (one a CU at least) have table entries for: the
+    pass takes the prefill tiles, as widths of partial units always did, and runs. One pair each stays on the GEMV."""
+    run_fake(tmp_path, f"""
+a = dict(hidden={H}, n_experts=1024, top_k=4, expert_ffn={F}, gate_type="Q8_0", down_type="Q8_0", max_tokens=1024)
+with layer(**a) as L:
+    for T, gemv in ((1024, False), (64, True)):
+        L.stage(np.zeros((T, {H}), np.uint16))
+        L.run()
+        assert ("router_quant" in L.kernel_names()) == gemv, (T, L.kernel_names())
+""")
