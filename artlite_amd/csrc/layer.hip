@@ -209,7 +209,7 @@ Path path_of(const artlite_moe_layer* L, int64_t T) {
   }
   p.shared_prefill = L->d.shared_ffn && p.prefill && L->shared_prefill_ok &&
                      T >= (p.stream && L->shared_stream_ok ? SHARED_STREAM + 1 : 64);
-  p.shared_stream = L->d.shared_ffn && !p.shared_gemv && !p.shared_prefill && L->shared_stream_ok;
+  p.shared_stream = L->d.shared_ffn && !p.shared_gemv && !p.shared_prefill && L->shared_stream_ok && T <= STREAM_FEW_ROWS;
   const bool planes = (!p.gemv && !p.prefill) || (L->d.shared_ffn && !p.shared_gemv && !p.shared_prefill);
   p.split = planes && (L->x_dtype == ARTLITE_X_F32 || L->d.norm_eps > 0);  // (the normalised x is fp32)
   p.quant = p.gemv;

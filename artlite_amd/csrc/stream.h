@@ -47,6 +47,9 @@ bool stream_supported(int qtype, int K, int N);
 // whether a launch of these takes every item of max_tiles tiles of bm rows
 bool stream_fits(int qtype, bool swiglu, int N, int bm, int64_t max_tiles);
 
+// the most rows of a launch of the dense rows (16 a step of the grid's second dimension)
+constexpr int STREAM_FEW_ROWS = 65535 * 16;
+
 int launch_stream(const StreamArgs& a, hipStream_t s);
 int launch_stream_few(const StreamFewArgs& a, hipStream_t s);
 

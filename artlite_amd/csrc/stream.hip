@@ -683,7 +683,7 @@ int launch_stream_few(const StreamFewArgs& a, hipStream_t s) {
   const bool swiglu = a.w[1] != nullptr;
   if (!stream_supported(a.qtype, a.K, a.N))
     return fail(ARTLITE_EINVAL, "streamed dense rows: weight type %d, K %d, N %d", a.qtype, a.K, a.N);
-  if (!a.w[0] || !a.a || (swiglu ? !a.h_hi || !a.h_lo : !a.y) || a.rows < 0 || a.rows > 65535 * 16)
+  if (!a.w[0] || !a.a || (swiglu ? !a.h_hi || !a.h_lo : !a.y) || a.rows < 0 || a.rows > STREAM_FEW_ROWS)
     return fail(ARTLITE_EINVAL, "streamed dense rows: null or mismatched argument");
   if (a.rows == 0) return ARTLITE_OK;
 #define ART_ST(QT) return swiglu ? launch_few<QT, true>(a, s) : launch_few<QT, false>(a, s)

@@ -32,3 +32,15 @@ with layer(**a) as L:
         L.run()
         assert ("router_quant" in L.kernel_names()) == gemv, (T, L.kernel_names())
 """)
+
+
+def test_shared_expert_of_a_million_tokens(tmp_path: Path) -> None:
+    """A shared expert narrower than the prefill tiles take, past the rows of one launch of the streamed dense rows."""
+    run_fake(tmp_path, """
+T = 65535 * 16 + 1
+with layer(hidden=64, n_experts=4, top_k=1, expert_ffn=64, gate_type="Q8_0", down_type="Q8_0", shared_ffn=64,
+           shared_type="Q8_0", max_tokens=T) as L:
+    for n in (T - 1, T):
+        L.stage(np.zeros((n, 64), np.uint16))
+        L.run()
+""")
