@@ -228,7 +228,7 @@ bool shared_dn_merged(const artlite_moe_layer* L, const Path& p) {
   return !p.stream && L->sdq && L->sdq->id == L->dq->id;
 }
 
-// the named kernels of a forward pass, in launch order
+// the named kernels of a forward pass, in launch order (the streamed tiles': '@' and their rows; the streamed dense rows')
 std::vector<std::string> kernel_list(const artlite_moe_layer* L, int64_t T) {
   const Path p = path_of(L, T);
   std::vector<std::string> k;
@@ -246,13 +246,14 @@ std::vector<std::string> kernel_list(const artlite_moe_layer* L, int64_t T) {
     k.push_back("dispatch_scatter");
   }
   const bool sp = p.prefill && p.shared_prefill;  // (the shared expert's items in the routed launches, or beside them)
-  k.push_back("gate_up");
+  const std::string tiles = p.stream ? "@stream" + std::to_string(p.stream) : "", rows = p.shared_stream ? "@stream" : "";
+  k.push_back("gate_up" + tiles);
   if (sp && !shared_gu_merged(L, p)) k.push_back("shared_gate_up");
-  k.push_back("down");
+  k.push_back("down" + tiles);
   if (sp && !shared_dn_merged(L, p)) k.push_back("shared_down");
   if (L->d.shared_ffn && !sp) {
-    k.push_back("shared_gate_up");
-    k.push_back("shared_down");
+    k.push_back("shared_gate_up" + rows);
+    k.push_back("shared_down" + rows);
   }
   k.push_back("combine");
   return k;

@@ -128,6 +128,7 @@ def time_T(gls: list, shape: dict, T: int, steps: int, warmup: int) -> dict:
         U.append(int((g.tap("counts") > 0).sum()))
         g.stage(x)
     mean, runs, kernels = time_layers(gls, warmup=warmup, iters=steps)
+    kernels = {n.split("@")[0]: v for n, v in kernels.items()}  # (a product's name without its variant)
     return {"ms": mean, "ms_median_evented": float(np.median(runs)), "kernels": kernels, "U": float(np.mean(U)),
             "names": list(kernels)}
 

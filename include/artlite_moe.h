@@ -157,7 +157,8 @@ int artlite_moe_layer_tap(artlite_moe_layer* layer, int tap, void* out, size_t n
  * average duration (artlite_moe_kernel_names order), kernel_cap entries at most; *n_kernels the count. */
 int artlite_moe_layer_time(artlite_moe_layer** layers, int n, int64_t T, int warmup, int iters, double* ms_per_run,
                            double* run_ms, double* kernel_ms, int kernel_cap, int* n_kernels);
-/* The names of the kernels of a run of T tokens on this layer, ';'-separated, into buf. */
+/* The names of the kernels of a run of T tokens on this layer, ';'-separated, into buf; a product's on the streamed tiles
+ * with '@' and their rows after it ("gate_up@stream16"), a shared expert's on the streamed dense rows with "@stream". */
 int artlite_moe_kernel_names(artlite_moe_layer* layer, int64_t T, char* buf, size_t cap);
 
 /* Bytes copied per ms by a plain device copy of nbytes (HBM calibration of the profile counters). */

@@ -28,8 +28,8 @@ CASES = [
     Spec("iq4_xs", H=512, E=8, k=2, F=512, gate_type="IQ4_XS", down_type="Q4_K", scale=5e-5, dmin_scale=1.5e-3),
 ]
 TOKENS = (17, 56, 57, 152)
-# (the formats with tiles of 64 rows: from 33 pairs per expert, up to 41, 45 and 54; then the first of the prefill tiles)
-LAST = {"q4_0": 41, "q8_0": 41, "q4_k": 45, "q8_0_only": 54}
+# (the formats with tiles of 64 rows: past 32 pairs per expert, up to 41, 45 and 54; then the first of the prefill tiles)
+LAST = {"Q4_0": 41, "Q4_K": 45, "Q8_0": 54}
 CASES_64 = [
     CASES[0], CASES[1],
     Spec("q4_k", H=512, E=8, k=2, F=512, gate_type="Q4_K", down_type="Q8_0", scale=2e-4, dmin_scale=1.5e-3),
@@ -41,9 +41,16 @@ SHARED = Spec("shared", H=512, E=16, k=2, F=384, gate_type="Q4_0", down_type="Q8
               shared_type="Q8_0", shared_down_type="Q4_0", shared_gated=True)
 
 
+def tiles(spec: Spec, T: int) -> str:
+    """The variant of the products' names that these cases are made for, by formats and pairs per expert."""
+    pairs, by64 = T * spec.k / spec.E, {spec.gate_type, spec.down_type} <= {"Q4_0", "Q4_K", "Q8_0"}
+    last = min(LAST[q] for q in (spec.gate_type, spec.down_type)) if by64 else 38
+    return "" if pairs > last else "@stream16" if pairs <= 14 else "@stream64" if by64 and pairs > 32 else "@stream32"
+
+
 @pytest.mark.parametrize(("spec", "tokens"),
                          [(s, TOKENS) for s in CASES]
-                         + [(s, (132, 133, LAST[s.name] * 4, LAST[s.name] * 4 + 1)) for s in CASES_64]
+                         + [(s, (128, 129, last := 4 * min(LAST[s.gate_type], LAST[s.down_type]), last + 1)) for s in CASES_64]
                          + [(replace(SHARED, x_dtype=x), (63, 64, 65, 256, 257)) for x in ("bf16", "f32")])
 def test_stream_tiles(spec: Spec, tokens: tuple) -> None:
     layer = layers.make_layer(spec, 7)
@@ -55,7 +62,8 @@ def test_stream_tiles(spec: Spec, tokens: tuple) -> None:
             x = np.abs(layers.make_x(spec, T, T))
             y = g(gpu_input(spec, x))
             names = g.kernel_names()
-            assert "prefill_x" in names and "router_quant" not in names, names
+            assert "prefill_x" in names and ("gate_up" + tiles(spec, T)) in names and ("down" + tiles(spec, T)) in names, names
+            assert not spec.shared_F or ("shared_down@stream" in names) == (T <= 256), names
             taps = check_against_oracle(g, layer, x, y)
             counts = g.tap("counts")
             # h and the pair outputs: fp16 x (fp32 x rounded once), h rounded once (2^-11 each at most)
