@@ -141,19 +141,48 @@ int check_ready(const artlite_moe_layer* L) {
 }
 
 // The prefill's routed products by the streamed small tiles (stream.hip): up to STREAM_16 pairs per expert on average in
-// tiles of 16 rows, up to STREAM_32 of 32, then of 64 in the formats that have them (Q4_0, Q4_K, Q8_0; in the others of 32
-// up to STREAM_32_ALONE), up to stream_last pairs: there the MFMA prefill tiles take over. Layer times in us (128 experts
-// 768 wide; 64 rows a tile / 32 / the prefill tiles):
+// tiles of 16 rows, then of 32 up to the formats' lines (stream_32; two formats: gate / up's two thirds of the weights take
+// two thirds of their line, the down a third) and STREAM_32_ALONE; where both formats have tiles of 64 rows, these past
+// STREAM_32 pairs up to stream_64. Past them the MFMA prefill tiles take over. The lines lie where the layer times of the
+// streamed tiles (first) and the prefill tiles meet, in us at the pairs given, of 128 experts 768 wide and of 32 experts 2816
+// wide (H 2048):
+//   Q6_K    19 220 / 246, 22 262 / 248          19 223 / 227, 22 246 / 228
+//   Q3_K    26 239 / 245, 28 261 / 247          26 222 / 231, 32 251 / 228
+//   Q5_K    32 232 / 249, 35 256 / 250          32 205 / 228, 38 237 / 227
+//   IQ4_XS  32 240 / 262, 35 269 / 265          32 218 / 241, 38 249 / 241
+//   Q4_1    35 245 / 251, 38 256 / 251          32 200 / 226, 38 231 / 227
+//   IQ4_NL  35 255 / 265, 38 266 / 264          32 220 / 241, 38 242 / 242
+//   Q4_K / Q6_K    36 263 / 279, 38 278 / 270   36 242 / 256, 38 250 / 252
+//   Q5_K / Q6_K    28 227 / 248, 31 250 / 248   25 226 / 228, 28 230 / 227
+//   Q3_K / Q4_K    31 256 / 278, 33 282 / 278   31 235 / 258, 33 248 / 258
+//   Q4_0 / Q6_K    31 226 / 230, 33 240 / 232   22 207 / 208, 28 212 / 210
+//   Q6_K / Q4_0    28 239 / 244, 31 268 / 245   25 206 / 227, 28 230 / 227
+// and of Q4_0, Q4_K and Q8_0 (128 experts 768 wide; 64 rows a tile / 32 / the prefill tiles):
 //   pairs      22               30               35               40               45               50
 //   Q4_0       174 / 170 / 221  190 / 188 / 224  205 / 219 / 228  213 / 242 / 229  250 / 248 / 233  261 / 253 / 234
 //   Q4_K       188 / 178 / 313  218 / 203 / 315  228 / 236 / 302  232 / 254 / 291  283 / 265 / 295  293 / 272 / 291
 //   Q8_0       213 / 220 / 288  238 / 237 / 289  246 / 272 / 290  251 / 298 / 289  275 / 305 / 292  277 / 315 / 294
 // (Q8_0 at 60 pairs 302 / 338 / 296; 32 experts 2880 wide in Q8_0 at 38 / 50 / 58 / 65 pairs 300 / 319 / 339 / 387 in
 // tiles of 64, 366 / 382 / 401 / 464 of 32, 383 / 383 / 385 / 386 on the prefill tiles. Q4_0 at 12.5 / 16 pairs in tiles
-// of 16 138 / 162, of 32 151 / 157.) A shared expert of the routed format joins the prefill tiles' launches and not these
-// (64 experts of Q4_K, 24 / 30 pairs, fp32 x: 259 / 300 against 306 / 294), so the line is lower there.
+// of 16 138 / 162, of 32 151 / 157. Q4_K's tiles of 32 are the fastest from 45 pairs on, which these lines leave unused.) A
+// shared expert of the routed format joins the prefill tiles' launches and not these (64 experts of Q4_K, 24 / 30 pairs, fp32
+// x: 259 / 300 against 306 / 294), so the line is STREAM_SHARED there at most.
 constexpr int STREAM_16 = 14, STREAM_32 = 32, STREAM_32_ALONE = 38, STREAM_SHARED = 28;
-constexpr int stream_last(int qtype) { return qtype == ARTLITE_Q8_0 ? 54 : qtype == ARTLITE_Q4_K ? 45 : 41; }
+constexpr int stream_32(int qtype) {
+  switch (qtype) {
+    case ARTLITE_Q4_K: return 45;
+    case ARTLITE_Q8_0: return 38;
+    case ARTLITE_IQ4_NL: return 37;
+    case ARTLITE_Q4_0:
+    case ARTLITE_Q4_1: return 36;
+    case ARTLITE_Q3_K: return 26;
+    case ARTLITE_Q6_K: return 20;
+    default: return 33;  // (Q5_K, IQ4_XS)
+  }
+}
+constexpr int stream_64(int qtype) {  // (0: no tiles of 64)
+  return qtype == ARTLITE_Q8_0 ? 54 : qtype == ARTLITE_Q4_K ? 45 : qtype == ARTLITE_Q4_0 ? 41 : 0;
+}
 
 // A shared expert beside streamed routed ones: up to this many tokens on the streamed dense rows, whose launches take its
 // few weight rows 16 tokens at a time, past them on launches of the prefill tiles. (2816 wide, Q4_K, the layer at 64 / 128
@@ -194,18 +223,17 @@ Path path_of(const artlite_moe_layer* L, int64_t T) {
   p.shared_gemv = L->d.shared_ffn && p.gemv && L->shared_gemv_ok;
   p.prefill = !p.gemv && L->prefill_ok;
   const bool joins = L->shared_prefill_ok && (L->sq->id == L->gq->id || L->sdq->id == L->dq->id);
-  const int last = joins ? STREAM_SHARED : std::min(stream_last(L->d.gate_type), stream_last(L->d.down_type));
-  if (p.prefill && L->stream_ok && P <= last * E) {
+  if (p.prefill && L->stream_ok && !(joins && P > STREAM_SHARED * E)) {
     const auto fits = [&](int bm) {
       const int64_t tiles = tile_bound(P, int(E), bm);
       return stream_fits(L->d.gate_type, true, L->d.expert_ffn, bm, tiles) &&
              stream_fits(L->d.down_type, false, L->d.hidden, bm, tiles);
     };
-    const int bm = P <= STREAM_16 * E ? 16 : P <= STREAM_32 * E ? 32 : 64;
-    if (fits(bm))
+    const int gq = L->d.gate_type, dq = L->d.down_type, bm = P <= STREAM_16 * E ? 16 : 32;
+    if (P > STREAM_32 * E && P <= std::min(stream_64(gq), stream_64(dq)) * E && fits(64))
+      p.stream = 64;
+    else if (P <= STREAM_32_ALONE * E && 3 * P <= (2 * stream_32(gq) + stream_32(dq)) * E && fits(bm))
       p.stream = bm;
-    else if (bm == 64 && P <= STREAM_32_ALONE * E && fits(32))
-      p.stream = 32;
   }
   p.shared_prefill = L->d.shared_ffn && p.prefill && L->shared_prefill_ok &&
                      T >= (p.stream && L->shared_stream_ok ? SHARED_STREAM + 1 : 64);

@@ -44,3 +44,17 @@ with layer(hidden=64, n_experts=4, top_k=1, expert_ffn=64, gate_type="Q8_0", dow
         L.stage(np.zeros((n, 64), np.uint16))
         L.run()
 """)
+
+
+@pytest.mark.parametrize(("gate", "down", "pairs"), [
+    ("Q6_K", "Q6_K", 20), ("Q3_K", "Q3_K", 26), ("Q5_K", "Q5_K", 33), ("IQ4_XS", "IQ4_XS", 33), ("Q4_1", "Q4_1", 36),
+    ("IQ4_NL", "IQ4_NL", 37), ("Q4_K", "Q6_K", 36), ("Q5_K", "Q6_K", 28), ("Q3_K", "Q4_K", 32), ("Q6_K", "Q4_0", 25),
+    ("Q4_K", "Q5_K", 38), ("Q4_0", "Q4_0", 41), ("Q4_K", "Q4_K", 45), ("Q8_0", "Q8_0", 54), ("Q4_0", "Q8_0", 41)])
+def test_streamed_lines(tmp_path: Path, gate: str, down: str, pairs: int) -> None:
+    """The last pairs an expert that stream, by the formats: past them the prefill tiles are faster."""
+    run_fake(tmp_path, f"""
+a = dict(hidden=2048, n_experts=128, top_k=8, expert_ffn=768, gate_type="{gate}", down_type="{down}")
+for p, stream in ((5, True), ({pairs}, True), ({pairs} + 1, False), (64, False)):
+    n = names(16 * p, **a)
+    assert any("gate_up@stream" in k for k in n) == stream, (p, n)
+""")
