@@ -141,22 +141,25 @@ int check_ready(const artlite_moe_layer* L) {
 }
 
 // The prefill's routed products by the streamed small tiles (stream.hip): up to STREAM_16 pairs per expert on average in
-// tiles of 16 rows, then of 32 up to the formats' lines (stream_32; two formats: gate / up's two thirds of the weights take
-// two thirds of their line, the down a third) and STREAM_32_ALONE; where both formats have tiles of 64 rows, these past
-// STREAM_32 pairs up to stream_64. Past them the MFMA prefill tiles take over. The lines lie where the layer times of the
-// streamed tiles (first) and the prefill tiles meet, in us at the pairs given, of 128 experts 768 wide and of 32 experts 2816
-// wide (H 2048):
-//   Q6_K    19 220 / 246, 22 262 / 248          19 223 / 227, 22 246 / 228
-//   Q3_K    26 239 / 245, 28 261 / 247          26 222 / 231, 32 251 / 228
-//   Q5_K    32 232 / 249, 35 256 / 250          32 205 / 228, 38 237 / 227
-//   IQ4_XS  32 240 / 262, 35 269 / 265          32 218 / 241, 38 249 / 241
-//   Q4_1    35 245 / 251, 38 256 / 251          32 200 / 226, 38 231 / 227
-//   IQ4_NL  35 255 / 265, 38 266 / 264          32 220 / 241, 38 242 / 242
-//   Q4_K / Q6_K    36 263 / 279, 38 278 / 270   36 242 / 256, 38 250 / 252
-//   Q5_K / Q6_K    28 227 / 248, 31 250 / 248   25 226 / 228, 28 230 / 227
-//   Q3_K / Q4_K    31 256 / 278, 33 282 / 278   31 235 / 258, 33 248 / 258
-//   Q4_0 / Q6_K    31 226 / 230, 33 240 / 232   22 207 / 208, 28 212 / 210
-//   Q6_K / Q4_0    28 239 / 244, 31 268 / 245   25 206 / 227, 28 230 / 227
+// tiles of 16 rows, then of 32 up to the formats' lines (stream_32) and STREAM_32_ALONE; where both formats have tiles of 64
+// rows, these past STREAM_32 pairs up to stream_64. Past them the MFMA prefill tiles take over. A line lies where the layer
+// times of the streamed tiles (first) and the prefill tiles meet, at the shape where that comes first, in us at the pairs
+// given; others meet up to 8 pairs later (H 2048: 32 x 1024 is 32 experts 1024 wide):
+//   Q6_K    128 x 768 19 220 / 246, 22 262 / 248   32 x 1024 18 106 / 113, 21 127 / 113   32 x 2816 21 224 / 228, 22 246 / 228
+//   Q3_K    128 x 768 26 239 / 245, 28 261 / 247   32 x 1024 22 104 / 110, 24 116 / 110   32 x 2048 22 154 / 171, 24 176 / 171
+//   Q5_K    128 x 768 32 232 / 249, 35 256 / 250   32 x 1024 32 107 / 114, 34 121 / 114   32 x 2816 32 205 / 228, 38 237 / 227
+//   IQ4_XS  128 x 768 32 240 / 262, 35 269 / 265   32 x 1024 32 115 / 118, 34 122 / 118   32 x 2816 32 218 / 241, 38 249 / 241
+//   Q4_1    128 x 768 35 245 / 251, 38 256 / 251   32 x 1024 32 105 / 113, 34 119 / 114   32 x 2816 32 200 / 226, 38 231 / 227
+//   IQ4_NL  128 x 768 35 255 / 265, 38 266 / 264   32 x 2816 32 220 / 241, 38 242 / 242
+// Of two formats, gate / up's two thirds of the weights take two thirds of their line and the down a third (Q4_K with a Q6_K
+// down, 128 x 768: 36 263 / 279, 38 278 / 270; Q3_K with Q4_K: 31 256 / 278, 33 282 / 278; Q6_K with Q4_0, 32 x 2816: 25 206 /
+// 227, 28 230 / 227), but a Q6_K down allows 22 pairs beside formats whose prefill tiles are faster than Q4_K's and Q8_0's
+// (Q4_0, 32 x 2816: 22 207 / 208, 28 212 / 210; 64 x 1024 of H 1024: 21 1.06 times as fast, 22 0.96). Two exceptions: layers
+// whose experts have at most 64 rows of gate and 128 of down a CU, one round of resident workgroups at two tiles an expert, in
+// which the tiles' own cost hides, stream to STREAM_32_ALONE in every format (16 x 1024 at 38 pairs: Q6_K 1.08, Q5_K 1.24
+// times as fast; 8 x 1024 of H 1024 1.11 to 1.45); and a shared expert that would take launches of its own beside prefill
+// tiles, and streams along, allows STREAM_OWN_SHARED pairs more (Q6_K, 32 x 2816 with one of 2816 in Q8_0, bf16 / fp32 x: 22
+// pairs 1.17 / 1.10, 26 0.99 / 0.94; Q3_K 28 1.08 / 1.02).
 // and of Q4_0, Q4_K and Q8_0 (128 experts 768 wide; 64 rows a tile / 32 / the prefill tiles):
 //   pairs      22               30               35               40               45               50
 //   Q4_0       174 / 170 / 221  190 / 188 / 224  205 / 219 / 228  213 / 242 / 229  250 / 248 / 233  261 / 253 / 234
@@ -167,17 +170,15 @@ int check_ready(const artlite_moe_layer* L) {
 // of 16 138 / 162, of 32 151 / 157. Q4_K's tiles of 32 are the fastest from 45 pairs on, which these lines leave unused.) A
 // shared expert of the routed format joins the prefill tiles' launches and not these (64 experts of Q4_K, 24 / 30 pairs, fp32
 // x: 259 / 300 against 306 / 294), so the line is STREAM_SHARED there at most.
-constexpr int STREAM_16 = 14, STREAM_32 = 32, STREAM_32_ALONE = 38, STREAM_SHARED = 28;
+constexpr int STREAM_16 = 14, STREAM_32 = 32, STREAM_32_ALONE = 38, STREAM_SHARED = 28, STREAM_OWN_SHARED = 6;
 constexpr int stream_32(int qtype) {
   switch (qtype) {
     case ARTLITE_Q4_K: return 45;
     case ARTLITE_Q8_0: return 38;
-    case ARTLITE_IQ4_NL: return 37;
-    case ARTLITE_Q4_0:
-    case ARTLITE_Q4_1: return 36;
-    case ARTLITE_Q3_K: return 26;
-    case ARTLITE_Q6_K: return 20;
-    default: return 33;  // (Q5_K, IQ4_XS)
+    case ARTLITE_IQ4_NL: return 34;
+    case ARTLITE_Q3_K: return 22;
+    case ARTLITE_Q6_K: return 19;
+    default: return 33;  // (Q4_0, Q4_1, Q5_K, IQ4_XS)
   }
 }
 constexpr int stream_64(int qtype) {  // (0: no tiles of 64)
@@ -189,6 +190,17 @@ constexpr int stream_64(int qtype) {  // (0: no tiles of 64)
 // / 256 / 320 tokens: 166 / 188 / 240 / 276 us against 223 / 235 / 280 / 289, in fp32 175 / 202 / 259 / 300 against 224 /
 // 233 / 281 / 289; 512 wide, Q8_0, 64 / 128 / 180 tokens: 76 / 83 / 87 against 113 / 120 / 123.)
 constexpr int64_t SHARED_STREAM = 256;
+
+// three times the pairs per expert up to which the routed products stream in tiles of at most 32 rows (own_shared: beside a
+// shared expert that streams along and would take prefill launches of its own)
+int64_t stream_line(const artlite_moe_layer* L, bool own_shared) {
+  const int gq = L->d.gate_type, dq = L->d.down_type;
+  const int64_t E = L->d.n_experts, most = 3 * STREAM_32_ALONE;
+  if (E * L->d.expert_ffn <= 64 * L->cus && E * L->d.hidden <= 128 * L->cus) return most;
+  int64_t line = 2 * stream_32(gq) + stream_32(dq);
+  if (dq == ARTLITE_Q6_K && gq != ARTLITE_Q4_K && gq != ARTLITE_Q8_0) line = std::min<int64_t>(line, 3 * 22);
+  return std::min(most, line + (own_shared ? 3 * STREAM_OWN_SHARED : 0));
+}
 
 // The kernels a forward pass of T tokens takes. Decode-sized passes (at most GEMV_BM pairs per expert on
 // average) run the experts on the VALU GEMV over XQ activations (it takes every block format); larger ones on the
@@ -229,10 +241,11 @@ Path path_of(const artlite_moe_layer* L, int64_t T) {
       return stream_fits(L->d.gate_type, true, L->d.expert_ffn, bm, tiles) &&
              stream_fits(L->d.down_type, false, L->d.hidden, bm, tiles);
     };
-    const int gq = L->d.gate_type, dq = L->d.down_type, bm = P <= STREAM_16 * E ? 16 : 32;
-    if (P > STREAM_32 * E && P <= std::min(stream_64(gq), stream_64(dq)) * E && fits(64))
+    const int bm = P <= STREAM_16 * E ? 16 : 32;
+    const bool own_shared = L->shared_stream_ok && !joins && T <= SHARED_STREAM;
+    if (P > STREAM_32 * E && P <= std::min(stream_64(L->d.gate_type), stream_64(L->d.down_type)) * E && fits(64))
       p.stream = 64;
-    else if (P <= STREAM_32_ALONE * E && 3 * P <= (2 * stream_32(gq) + stream_32(dq)) * E && fits(bm))
+    else if (3 * P <= stream_line(L, own_shared) * E && fits(bm))
       p.stream = bm;
   }
   p.shared_prefill = L->d.shared_ffn && p.prefill && L->shared_prefill_ok &&

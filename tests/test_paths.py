@@ -47,14 +47,22 @@ with layer(hidden=64, n_experts=4, top_k=1, expert_ffn=64, gate_type="Q8_0", dow
 
 
 @pytest.mark.parametrize(("gate", "down", "pairs"), [
-    ("Q6_K", "Q6_K", 20), ("Q3_K", "Q3_K", 26), ("Q5_K", "Q5_K", 33), ("IQ4_XS", "IQ4_XS", 33), ("Q4_1", "Q4_1", 36),
-    ("IQ4_NL", "IQ4_NL", 37), ("Q4_K", "Q6_K", 36), ("Q5_K", "Q6_K", 28), ("Q3_K", "Q4_K", 32), ("Q6_K", "Q4_0", 25),
-    ("Q4_K", "Q5_K", 38), ("Q4_0", "Q4_0", 41), ("Q4_K", "Q4_K", 45), ("Q8_0", "Q8_0", 54), ("Q4_0", "Q8_0", 41)])
+    ("Q6_K", "Q6_K", 19), ("Q3_K", "Q3_K", 22), ("Q5_K", "Q5_K", 33), ("IQ4_XS", "IQ4_XS", 33), ("Q4_1", "Q4_1", 33),
+    ("IQ4_NL", "IQ4_NL", 34), ("Q4_K", "Q6_K", 36), ("Q5_K", "Q6_K", 22), ("Q4_0", "Q6_K", 22), ("Q3_K", "Q4_K", 29),
+    ("Q6_K", "Q4_0", 23), ("Q4_K", "Q5_K", 38), ("Q4_0", "Q4_0", 41), ("Q4_K", "Q4_K", 45), ("Q8_0", "Q8_0", 54),
+    ("Q4_0", "Q8_0", 41)])
 def test_streamed_lines(tmp_path: Path, gate: str, down: str, pairs: int) -> None:
-    """The last pairs an expert that stream, by the formats: past them the prefill tiles are faster."""
+    """The last pairs an expert that stream, by the formats: past them the prefill tiles are faster. Layers of few rows
+    stream to 38 at least in every format; a shared expert of another format, while it streams along, adds six."""
     run_fake(tmp_path, f"""
-a = dict(hidden=2048, n_experts=128, top_k=8, expert_ffn=768, gate_type="{gate}", down_type="{down}")
-for p, stream in ((5, True), ({pairs}, True), ({pairs} + 1, False), (64, False)):
-    n = names(16 * p, **a)
-    assert any("gate_up@stream" in k for k in n) == stream, (p, n)
+def streams(T, **a): return any("gate_up@stream" in k for k in names(T, hidden=2048, gate_type="{gate}", down_type="{down}", **a))
+for p, want in ((5, True), ({pairs}, True), ({pairs} + 1, False), (64, False)):
+    assert streams(16 * p, n_experts=128, top_k=8, expert_ffn=768) == want, p
+few = max({pairs}, 38)
+for p, want in ((20, True), (few, True), (few + 1, False)):
+    assert streams(8 * p, n_experts=16, top_k=2, expert_ffn=1024) == want, p
+other = "Q4_1" if "{gate}" != "Q4_1" != "{down}" else "Q4_0"
+own = dict(n_experts=128, top_k=32, expert_ffn=768, shared_ffn=512, shared_type=other)
+for p, want in (({pairs} + 1, True), ({pairs} + 5 if {pairs} < 33 else 38, True), (max({pairs}, 38) + 1, False)):
+    assert {pairs} >= 38 or streams(4 * p, **own) == want, p
 """)

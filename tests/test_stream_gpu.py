@@ -15,7 +15,7 @@ from .helpers import check_against_oracle, check_pairs_f64, gpu_input, gpu_layer
 pytestmark = pytest.mark.gpu
 
 Spec = layers.Spec
-# (hidden and expert width; token counts: more than 4 pairs per expert, up to 14 (tiles of 16 rows), up to the formats' lines)
+# (hidden and expert width; token counts: more than 4 pairs per expert, up to 14 (tiles of 16 rows), up to 38 (of 32))
 CASES = [
     Spec("q4_0", H=448, E=8, k=2, F=336 + 48, gate_type="Q4_0", down_type="Q8_0", scale=0.02),
     Spec("q8_0", H=576, E=8, k=2, F=320, gate_type="Q8_0", down_type="Q4_0", scale=0.01, x_dtype="f32"),
@@ -27,16 +27,8 @@ CASES = [
     Spec("q3_k", H=512, E=8, k=2, F=512, gate_type="Q3_K", down_type="Q5_K", scale=1e-4, dmin_scale=1e-3),
     Spec("iq4_xs", H=512, E=8, k=2, F=512, gate_type="IQ4_XS", down_type="Q4_K", scale=5e-5, dmin_scale=1.5e-3),
 ]
-# pairs per expert that the formats stream up to in tiles of 32 rows (two formats: two thirds of gate / up's and a third of the
-# down's, 38 at most), and the formats with tiles of 64 rows up to: past 32 pairs per expert
-LAST_32 = {"Q4_K": 45, "Q8_0": 38, "IQ4_NL": 37, "Q4_0": 36, "Q4_1": 36, "Q5_K": 33, "IQ4_XS": 33, "Q3_K": 26, "Q6_K": 20}
-LAST_64 = {"Q4_0": 41, "Q4_K": 45, "Q8_0": 54}
-
-
-def last_32(s: Spec) -> int:
-    return min(38, (2 * LAST_32[s.gate_type] + LAST_32[s.down_type]) // 3)
-
-
+# (pairs per expert that layers of this size stream up to in tiles of 32 rows, and the formats with tiles of 64 past 32 pairs)
+LAST_32, LAST_64 = 38, {"Q4_0": 41, "Q4_K": 45, "Q8_0": 54}
 CASES_64 = [
     CASES[0], CASES[1],
     Spec("q4_k", H=512, E=8, k=2, F=512, gate_type="Q4_K", down_type="Q8_0", scale=2e-4, dmin_scale=1.5e-3),
@@ -53,11 +45,11 @@ def tiles(spec: Spec, T: int) -> str:
     pairs, by64 = T * spec.k / spec.E, {spec.gate_type, spec.down_type} <= set(LAST_64)
     if by64 and pairs > 32:
         return "@stream64" if pairs <= min(LAST_64[spec.gate_type], LAST_64[spec.down_type]) else ""
-    return "" if pairs > last_32(spec) else "@stream16" if pairs <= 14 else "@stream32"
+    return "" if pairs > LAST_32 else "@stream16" if pairs <= 14 else "@stream32"
 
 
 @pytest.mark.parametrize(("spec", "tokens"),
-                         [(s, (17, 56, 57, 4 * last_32(s))) for s in CASES]
+                         [(s, (17, 56, 57, 4 * LAST_32)) for s in CASES]
                          + [(s, (128, 129, n := 4 * min(LAST_64[s.gate_type], LAST_64[s.down_type]), n + 1)) for s in CASES_64]
                          + [(replace(SHARED, x_dtype=x), (63, 64, 65, 256, 257)) for x in ("bf16", "f32")])
 def test_stream_tiles(spec: Spec, tokens: tuple) -> None:
