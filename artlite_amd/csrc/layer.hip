@@ -190,6 +190,27 @@ constexpr int stream_64(int qtype) {  // (0: no tiles of 64)
 // / 256 / 320 tokens: 166 / 188 / 240 / 276 us against 223 / 235 / 280 / 289, in fp32 175 / 202 / 259 / 300 against 224 /
 // 233 / 281 / 289; 512 wide, Q8_0, 64 / 128 / 180 tokens: 76 / 83 / 87 against 113 / 120 / 123.)
 constexpr int64_t SHARED_STREAM = 256;
+// A shared expert of the routed format joins the prefill tiles' launches from 64 tokens on, which costs it little. Streamed,
+// it costs by its tokens (twice in fp32, two planes) times its share of the routed weights, r = T Fs / (E F): what a format's
+// rows take of what streaming the routed experts saves, in thousandths at r = 1 (2/3 gate and up's, 1/3 the down's). Layer
+// times streamed / on the prefill tiles, 16 experts 1024 wide with one of 2048, at r (fp32: 2 r):
+//   Q4_K 28 124 / 142, fp32 56 137 / 139     Q8_0 28 125 / 140, fp32 50 135 / 137, 56 142 / 140
+//   Q4_0 28 120 / 131, fp32 50 124 / 128, 56 132 / 129 (8 experts 1536 wide, one of 3072: fp32 32 108 / 117, 40 121 / 119)
+//   Q5_K 28 128 / 130, fp32 40 119 / 123, 50 135 / 133     Q4_1 28 126 / 133, fp32 40 121 / 125, 50 135 / 133
+//   Q3_K 10 97 / 110, 16 112 / 116, fp32 16 98 / 108, 24 125 / 111
+//   Q6_K 14 111 / 115, 16 125 / 116, fp32 16 98 / 111, 24 121 / 113
+// Routed experts of Q6_K and Q3_K, whose lines are early, save half as much past tiles of 16 rows (64 experts 1280 wide with
+// one of 2816, Q6_K at 15 pairs: r 5.5 251 / 272, fp32 11 279 / 271).
+constexpr int stream_shared_cost(int qtype) {
+  switch (qtype) {
+    case ARTLITE_Q3_K:
+    case ARTLITE_Q6_K: return 62;
+    case ARTLITE_Q4_0:
+    case ARTLITE_Q4_1:
+    case ARTLITE_Q5_K: return 25;
+    default: return 20;  // (Q4_K, Q8_0, IQ4_NL, IQ4_XS)
+  }
+}
 
 // three times the pairs per expert up to which the routed products stream in tiles of at most 32 rows (own_shared: beside a
 // shared expert that streams along and would take prefill launches of its own)
@@ -200,6 +221,17 @@ int64_t stream_line(const artlite_moe_layer* L, bool own_shared) {
   int64_t line = 2 * stream_32(gq) + stream_32(dq);
   if (dq == ARTLITE_Q6_K && gq != ARTLITE_Q4_K && gq != ARTLITE_Q8_0) line = std::min<int64_t>(line, 3 * 22);
   return std::min(most, line + (own_shared ? 3 * STREAM_OWN_SHARED : 0));
+}
+
+// whether T tokens of a shared expert that would join the prefill launches cost less streamed than the routed experts save
+bool shared_streams(const artlite_moe_layer* L, int64_t T) {
+  if (T < 64) return true;  // (too few for the prefill tiles)
+  const artlite_moe_desc& d = L->d;
+  const int planes = L->x_dtype == ARTLITE_X_F32 || d.norm_eps > 0 ? 2 : 1;
+  const bool early = 2 * stream_32(d.gate_type) + stream_32(d.down_type) < 3 * 25;
+  const int64_t saved = early && T * d.top_k > STREAM_16 * d.n_experts ? 500 : 1000;
+  return planes * T * d.shared_ffn * (2 * stream_shared_cost(L->sq->id) + stream_shared_cost(L->sdq->id)) <=
+         3 * saved * d.n_experts * d.expert_ffn;
 }
 
 // The kernels a forward pass of T tokens takes. Decode-sized passes (at most GEMV_BM pairs per expert on
@@ -235,7 +267,8 @@ Path path_of(const artlite_moe_layer* L, int64_t T) {
   p.shared_gemv = L->d.shared_ffn && p.gemv && L->shared_gemv_ok;
   p.prefill = !p.gemv && L->prefill_ok;
   const bool joins = L->shared_prefill_ok && (L->sq->id == L->gq->id || L->sdq->id == L->dq->id);
-  if (p.prefill && L->stream_ok && !(joins && P > STREAM_SHARED * E)) {
+  const bool join = joins && (P > STREAM_SHARED * E || (T <= SHARED_STREAM && !shared_streams(L, T)));
+  if (p.prefill && L->stream_ok && !join) {
     const auto fits = [&](int bm) {
       const int64_t tiles = tile_bound(P, int(E), bm);
       return stream_fits(L->d.gate_type, true, L->d.expert_ffn, bm, tiles) &&

@@ -66,3 +66,18 @@ own = dict(n_experts=128, top_k=32, expert_ffn=768, shared_ffn=512, shared_type=
 for p, want in (({pairs} + 1, True), ({pairs} + 5 if {pairs} < 33 else 38, True), (max({pairs}, 38) + 1, False)):
     assert {pairs} >= 38 or streams(4 * p, **own) == want, p
 """)
+
+
+@pytest.mark.parametrize(("fmt", "down", "x", "last"), [
+    ("Q6_K", "Q6_K", "bf16", 112), ("Q6_K", "Q6_K", "f32", 64), ("Q3_K", "Q3_K", "f32", 64), ("Q4_K", "Q6_K", "f32", 112),
+    ("Q5_K", "Q6_K", "f32", 96), ("Q5_K", "Q5_K", "f32", 160), ("Q4_0", "Q4_0", "bf16", 224), ("Q4_K", "Q4_K", "f32", 200)])
+def test_streamed_shared_expert(tmp_path: Path, fmt: str, down: str, x: str, last: int) -> None:
+    """The last tokens (of these) at which 16 experts 1024 wide stream beside a shared one of 2048 of their formats: past
+    them it is faster to join the prefill tiles' launches. Below 64 tokens it streams in any case."""
+    run_fake(tmp_path, f"""
+a = dict(hidden=2048, n_experts=16, top_k=2, expert_ffn=1024, gate_type="{fmt}", down_type="{down}", shared_ffn=2048,
+         shared_type="{fmt}", shared_down_type="{down}")
+for T in (33, 63, 64, 80, 96, 112, 128, 160, 200, 224, 225):
+    n = names(T, "{x}", **a)
+    assert any("@stream" in k for k in n) == (T <= {last}) == ("shared_down@stream" in n), (T, n)
+""")
