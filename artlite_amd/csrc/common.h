@@ -58,14 +58,14 @@ struct DevBuf {
 struct PinBuf {
   void* p = nullptr;
   size_t n = 0;
-  int reserve(size_t bytes);  // does not keep the contents
+  bool reserve(size_t bytes);  // does not keep the contents; false: none to be had (no error is left behind)
   void release();
   template <class T>
   T* as() const { return static_cast<T*>(p); }
   ~PinBuf() { release(); }
 };
-// The most that a host-pointer call stages each way through its thread's pinned buffers; larger arrays go by pageable
-// copies. (A pageable copy and its synchronization cost 15 to 30 us however small: 16 fp32 tokens of 1024 values through a
+// The most that a host-pointer call stages each way through its thread's pinned buffers; larger arrays, and all where no
+// pinned memory is to be had, go by pageable copies. (A pageable copy and its synchronization cost 15 to 30 us however small: 16 fp32 tokens of 1024 values through a
 // layer took 129 us with three of them, of which its kernels 51.)
 constexpr size_t PIN_MAX = size_t(4) << 20;
 
@@ -76,6 +76,10 @@ struct HostCtx {
   hipStream_t stream = nullptr;
   DevBuf in, out, out2, out3, out4, out5, tmp, tmp2, flag;
   PinBuf pin_in, pin_out;
+  // both buffers for calls of at most PIN_MAX each way (false: pageable copies)
+  bool pins(size_t in, size_t out) {
+    return in <= PIN_MAX && out <= PIN_MAX && pin_in.reserve(in) && pin_out.reserve(out);
+  }
 };
 int host_ctx(HostCtx** ctx);
 

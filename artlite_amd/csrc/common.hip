@@ -70,16 +70,18 @@ void DevBuf::release() {
   n = 0;
 }
 
-int PinBuf::reserve(size_t bytes) {
-  if (bytes <= n && p) return ARTLITE_OK;
+bool PinBuf::reserve(size_t bytes) {
+  if (bytes <= n && p) return true;
   release();
   const size_t want = (bytes + 65536) / 65536 * 65536;
   void* q = nullptr;
-  hipError_t e = hipHostMalloc(&q, want, hipHostMallocDefault);
-  if (e != hipSuccess) return fail(ARTLITE_ENOMEM, "hipHostMalloc(%zu): %s", want, hipGetErrorString(e));
+  if (hipHostMalloc(&q, want, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();  // (else the next launch's check would find it)
+    return false;
+  }
   p = q;
   n = want;
-  return ARTLITE_OK;
+  return true;
 }
 
 void PinBuf::release() {

@@ -418,9 +418,7 @@ extern "C" int artlite_moe_plan(const int32_t* ids, int64_t n, int k, int E, int
   PlanMem m{c->in.as<int32_t>(), c->out.as<int32_t>(), c->out2.as<int32_t>(), c->out3.as<int32_t>(),
             c->out5.as<int32_t>() + CTRL_BYTES / 4, c->out5.as<int32_t>(), c->out4.as<int64_t>()};
   const size_t back = CTRL_BYTES + b[5] + 16 + b[4];
-  if (b[0] <= PIN_MAX && back <= PIN_MAX) {
-    ART_TRY(c->pin_in.reserve(b[0]));
-    ART_TRY(c->pin_out.reserve(back));
+  if (c->pins(b[0], back)) {
     m.pin_in = c->pin_in.as<uint8_t>();
     m.pin_out = c->pin_out.as<uint8_t>();
   }

@@ -1041,12 +1041,10 @@ extern "C" int artlite_moe_layer_forward(artlite_moe_layer* L, const void* x, in
   ART_TRY(check_stage(L, x, x_dtype, T));
   const size_t xb = size_t(T) * L->d.hidden * (x_dtype == ARTLITE_X_F32 ? 4 : 2), yb = size_t(T) * L->d.hidden * 4;
   constexpr size_t CB = (CTRL_WORDS * 4 + 15) / 16 * 16;
-  if (T > 0 && y && xb <= PIN_MAX && CB + yb <= PIN_MAX) {  // (through the thread's pinned buffers: one synchronization)
+  HostCtx* c = nullptr;
+  if (T > 0 && y && xb <= PIN_MAX && CB + yb <= PIN_MAX) ART_TRY(host_ctx(&c));
+  if (c && c->pins(xb, CB + yb)) {  // (through the thread's pinned buffers: one synchronization)
     ART_TRY(check_ready(L));
-    HostCtx* c;
-    ART_TRY(host_ctx(&c));
-    ART_TRY(c->pin_in.reserve(xb));
-    ART_TRY(c->pin_out.reserve(CB + yb));
     std::memcpy(c->pin_in.p, x, xb);
     ART_TRY(launch_copy2(L->x.p, c->pin_in.p, xb, nullptr, nullptr, 0, nullptr, 0, L->stream));
     L->x_dtype = x_dtype;

@@ -725,9 +725,7 @@ namespace {
 int route_host(HostCtx* c, const float* logits, size_t need, int64_t n, int64_t row, int64_t ext, int per_col,
                int64_t pitch, int E, int k, int sigmoid, int32_t* ids, float* w32, double* w64) {
   const size_t nk = size_t(n) * k, wb = w64 ? 8 : 4;
-  if (need * 4 <= PIN_MAX && nk * (4 + wb) + 16 <= PIN_MAX) {
-    ART_TRY(c->pin_in.reserve(need * 4));
-    ART_TRY(c->pin_out.reserve(nk * (4 + wb) + 16));
+  if (c->pins(need * 4, nk * (4 + wb) + 16)) {
     float* in = c->pin_in.as<float>();
     uint8_t* wo = c->pin_out.as<uint8_t>();  // (the weights, then the ids)
     int32_t* io = reinterpret_cast<int32_t*>(wo + nk * wb);

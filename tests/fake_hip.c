@@ -1,10 +1,11 @@
 /* A stand-in for the HIP runtime on the CPU, for tests of the library's host code: allocations are untouched address
- * space, copies and fills do nothing, launches are counted, and one of them or the pinned allocations can be made to
- * fail. No kernel runs, so no result means anything. A 256-CU device that holds fake_per_cu workgroups of any kernel a
+ * space, copies and fills do nothing (what comes to the host is zeros), launches are counted, and one of them or the pinned
+ * allocations can be made to fail. No kernel runs, so no result means anything. A 256-CU device that holds fake_per_cu workgroups of any kernel a
  * CU. Loaded with RTLD_GLOBAL before the library, whose HIP calls then land here. */
 #define _GNU_SOURCE
 #include <stddef.h>
 #include <stdint.h>
+#include <string.h>
 #include <sys/mman.h>
 
 typedef struct { uint32_t x, y, z; } dim3;
@@ -35,16 +36,21 @@ int hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void* f, int thre
 int hipGetSymbolAddress(void** p, const void* symbol) { return (void)symbol, map(p, 8 << 20); }
 int hipMalloc(void** p, size_t n) { return fake_mallocs++, map(p, n); }
 int hipFree(void* p) { return (void)p, OK; }
-int hipHostMalloc(void** p, size_t n, unsigned flags) { return (void)flags, fake_fail_host_malloc ? NOMEM : map(p, n); }
+int hipHostMalloc(void** p, size_t n, unsigned flags) {
+  return (void)flags, fake_fail_host_malloc ? (last_error = NOMEM) : map(p, n);
+}
 int hipHostFree(void* p) { return (void)p, fake_freed_busy += fake_pending != 0, OK; }
 int hipStreamCreateWithFlags(stream_t* s, unsigned flags) {
   return (void)flags, *s = (stream_t)(uintptr_t)(++fake_streams), OK;
 }
 int hipStreamDestroy(stream_t s) { return (void)s, OK; }
 int hipStreamSynchronize(stream_t s) { return fake_pending -= pending_of[slot(s)], pending_of[slot(s)] = 0, OK; }
-int hipMemcpy(void* d, const void* s, size_t n, int kind) { return (void)d, (void)s, (void)n, (void)kind, fake_copies++, OK; }
+int hipMemcpy(void* d, const void* s, size_t n, int kind) {
+  if (kind == 2 /* to the host */) memset(d, 0, n);
+  return (void)s, fake_copies++, OK;
+}
 int hipMemcpyAsync(void* d, const void* src, size_t n, int kind, stream_t s) {
-  return (void)d, (void)src, (void)n, (void)kind, fake_copies++, queued(s), OK;
+  return queued(s), hipMemcpy(d, src, n, kind);
 }
 int hipMemsetAsync(void* d, int v, size_t n, stream_t s) { return (void)d, (void)v, (void)n, queued(s), OK; }
 int hipMemsetD32Async(void* d, int v, size_t n, stream_t s) { return (void)d, (void)v, (void)n, queued(s), OK; }

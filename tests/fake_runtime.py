@@ -1,6 +1,6 @@
 """Host code of the library on the CPU: a snippet run in a process of its own, where the library's HIP calls land in
 ``fake_hip.c``. It sees ``hip`` (the stand-in's counters and switches: ``hip.launches`` ..), ``_hip``, ``np``, ``MR``
-(routing), ``Plan``, ``MoELayer`` and ``layer(ready=True, **args)`` (a layer, by default with every tensor uploaded:
+(routing), ``route``, ``Plan``, ``MoELayer`` and ``layer(ready=True, **args)`` (a layer, by default with every tensor uploaded:
 untouched zeros)."""
 
 import subprocess
@@ -21,7 +21,7 @@ from artlite_amd import _hip
 from artlite_amd.gguf_model import TYPE_ID
 from artlite_amd.moe import route as MR
 from artlite_amd.moe.layer import TENSORS, MoELayer
-from artlite_amd.moe.plan import Plan
+from artlite_amd.moe.plan import Plan, route
 BLOCK = dict(Q4_0=(32, 18), Q4_1=(32, 20), Q8_0=(32, 34), Q3_K=(256, 110), Q4_K=(256, 144), Q5_K=(256, 176),
              Q6_K=(256, 210), IQ4_NL=(32, 18), IQ4_XS=(256, 136))
 def layer(ready=True, **a):

@@ -1,0 +1,28 @@
+"""The host-pointer calls' own errors and fall-backs, on the CPU (no kernel runs)."""
+
+from pathlib import Path
+
+from .fake_runtime import run_fake
+
+CALLS = """
+L = layer(hidden=1024, n_experts=8, top_k=2, expert_ffn=512, gate_type="Q8_0", down_type="Q8_0", max_tokens=64)
+logits, x = np.zeros((5000, 128), np.float32), np.zeros((40, 1024), np.float32)
+CALLS = dict(route=lambda: route(logits, 8), top_k=lambda: MR.top_k(logits, 8),
+             plan=lambda: Plan.of(np.zeros((500, 8), np.int32), cap=200, E=128), layer=lambda: L(x))
+"""
+
+
+def test_without_pinned_memory(tmp_path: Path) -> None:
+    """Where no pinned memory is to be had the calls take pageable copies, as they do beyond the pinned buffers' size."""
+    run_fake(tmp_path, CALLS + """
+hip.fail_host_malloc = 1
+for name, call in CALLS.items():
+    before = hip.copies
+    call()
+    assert hip.copies >= before + 2, name  # (to the device and back)
+hip.fail_host_malloc = 0
+for name, call in CALLS.items():
+    before = hip.copies
+    call()
+    assert hip.copies == before, name
+""")
