@@ -83,6 +83,16 @@ struct HostCtx {
 };
 int host_ctx(HostCtx** ctx);
 
+// Waits for a stream at the end of its scope while `on`: a call that has queued work on the thread's pinned buffers does not
+// return before that has run, whichever way it ends (the next call writes and may free them).
+struct Drain {
+  hipStream_t s;
+  bool on = true;
+  ~Drain() {
+    if (on) (void)hipStreamSynchronize(s);
+  }
+};
+
 // Copies on the stream by a kernel, between device memory and pinned host memory, whole 4-byte words each: n0 bytes of s0
 // to d0, then (n1 > 0) n1 bytes of s1 to d1, and (zero_words) zeros to that many words of z. A kernel and not a copy
 // engine's transfer, so that the launches around it follow in order with no signal between engines.

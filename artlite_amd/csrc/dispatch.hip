@@ -320,6 +320,7 @@ int plan_run(const int32_t* ids, int64_t n, int k, int E, int cols, int cap, int
              int32_t* counts, int32_t* sizes, int32_t* rows, int64_t* pos, const PlanMem& m, hipStream_t s) {
   const int64_t P = n * k;
   const size_t slots = size_t(cols) * cap;
+  Drain drain{s, m.pin_in != nullptr};
   const size_t o5_bytes = (slots * chunk + 2 * slots + cols) * 4, o5_pad = (o5_bytes + 15) / 16 * 16;
   if (m.pin_in) {
     if (P) std::memcpy(m.pin_in, ids, size_t(P) * 4);
@@ -342,6 +343,7 @@ int plan_run(const int32_t* ids, int64_t n, int k, int E, int cols, int cap, int
     from = PlanBufs{cols, cap, o5 + slots * chunk, o5 + slots * chunk + 2 * slots, o5 + slots * chunk + slots, o5,
                     reinterpret_cast<int64_t*>(m.pin_out + CTRL_BYTES + o5_pad)};
     ART_HIP(hipStreamSynchronize(s));
+    drain.on = false;
     std::memcpy(ctrl, m.pin_out, sizeof ctrl);
   } else {
     ART_HIP(hipMemcpyAsync(ctrl, m.ctrl, sizeof ctrl, hipMemcpyDeviceToHost, s));

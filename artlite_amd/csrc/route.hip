@@ -726,6 +726,7 @@ int route_host(HostCtx* c, const float* logits, size_t need, int64_t n, int64_t 
                int64_t pitch, int E, int k, int sigmoid, int32_t* ids, float* w32, double* w64) {
   const size_t nk = size_t(n) * k, wb = w64 ? 8 : 4;
   if (c->pins(need * 4, nk * (4 + wb) + 16)) {
+    Drain drain{c->stream};
     float* in = c->pin_in.as<float>();
     uint8_t* wo = c->pin_out.as<uint8_t>();  // (the weights, then the ids)
     int32_t* io = reinterpret_cast<int32_t*>(wo + nk * wb);
@@ -740,6 +741,7 @@ int route_host(HostCtx* c, const float* logits, size_t need, int64_t n, int64_t 
                           w64 ? reinterpret_cast<double*>(wo) + t * k : nullptr, c->stream));
     }
     ART_HIP(hipStreamSynchronize(c->stream));
+    drain.on = false;
     std::memcpy(ids, io, nk * 4);
     std::memcpy(w64 ? static_cast<void*>(w64) : static_cast<void*>(w32), wo, nk * wb);
     return ARTLITE_OK;

@@ -26,3 +26,34 @@ for name, call in CALLS.items():
     call()
     assert hip.copies == before, name
 """)
+
+
+def test_failed_launch_leaves_nothing_queued(tmp_path: Path) -> None:
+    """Whichever launch of a call fails, what was queued on the thread's pinned buffers before it has run when the call
+    returns: the next call writes them, and may free them for larger ones."""
+    run_fake(tmp_path, CALLS + """
+for name, call in CALLS.items():
+    before = hip.launches
+    call()
+    n = hip.launches - before
+    assert n >= 2 and hip.pending == 0, (name, n)
+    for i in range(n):
+        hip.fail_launch = hip.launches + i
+        try:
+            call()
+        except _hip.Error as e:
+            assert "invalid" in str(e), e
+        else:
+            raise AssertionError((name, i))
+        assert hip.pending == 0, (name, i, n)
+    hip.fail_launch = -1
+    call()
+L.close()
+L = layer(hidden=1024, n_experts=8, top_k=2, expert_ffn=512, gate_type="Q8_0", down_type="Q8_0", max_tokens=512)
+hip.fail_launch = hip.launches + 3
+try: L(x)
+except _hip.Error: pass
+hip.fail_launch = -1
+L(np.zeros((512, 1024), np.float32))  # (larger buffers: the others are freed)
+assert hip.freed_busy == 0
+""")
