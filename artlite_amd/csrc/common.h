@@ -81,7 +81,7 @@ struct HostCtx {
     return in <= PIN_MAX && out <= PIN_MAX && pin_in.reserve(in) && pin_out.reserve(out);
   }
 };
-int host_ctx(HostCtx** ctx);
+int host_ctx(HostCtx** ctx, bool stream = true);  // (stream false: for the buffers alone)
 
 // Waits for a stream at the end of its scope while `on`: a call that has queued work on the thread's pinned buffers does not
 // return before that has run, whichever way it ends (the next call writes and may free them).

@@ -104,7 +104,7 @@ struct CtxHolder {
 thread_local CtxHolder g_ctx;
 }  // namespace
 
-int host_ctx(HostCtx** out) {
+int host_ctx(HostCtx** out, bool stream) {
   int n = 0;
   hipError_t e = hipGetDeviceCount(&n);
   if (e != hipSuccess || n == 0) return fail(ARTLITE_EHIP, "no HIP device (hipGetDeviceCount: %s)", hipGetErrorString(e));
@@ -115,8 +115,8 @@ int host_ctx(HostCtx** out) {
   if (!c) {
     c = new HostCtx();
     c->device = dev;
-    ART_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   }
+  if (stream && !c->stream) ART_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   *out = c;
   return ARTLITE_OK;
 }

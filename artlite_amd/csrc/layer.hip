@@ -1042,7 +1042,7 @@ extern "C" int artlite_moe_layer_forward(artlite_moe_layer* L, const void* x, in
   const size_t xb = size_t(T) * L->d.hidden * (x_dtype == ARTLITE_X_F32 ? 4 : 2), yb = size_t(T) * L->d.hidden * 4;
   constexpr size_t CB = (CTRL_WORDS * 4 + 15) / 16 * 16;
   HostCtx* c = nullptr;
-  if (T > 0 && y && xb <= PIN_MAX && CB + yb <= PIN_MAX) ART_TRY(host_ctx(&c));
+  if (T > 0 && y && xb <= PIN_MAX && CB + yb <= PIN_MAX) ART_TRY(host_ctx(&c, false));
   if (c && c->pins(xb, CB + yb)) {  // (through the thread's pinned buffers: one synchronization)
     ART_TRY(check_ready(L));
     Drain drain{L->stream};

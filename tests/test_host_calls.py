@@ -57,3 +57,15 @@ hip.fail_launch = -1
 L(np.zeros((512, 1024), np.float32))  # (larger buffers: the others are freed)
 assert hip.freed_busy == 0
 """)
+
+
+def test_layer_call_makes_no_stream(tmp_path: Path) -> None:
+    """A layer's call runs on the layer's own stream: the thread's is made by the first call that needs it."""
+    run_fake(tmp_path, CALLS + """
+assert hip.streams == 1
+L(x)
+assert hip.streams == 1
+CALLS["route"]()
+CALLS["plan"]()
+assert hip.streams == 2
+""")
