@@ -1044,12 +1044,12 @@ extern "C" int artlite_moe_layer_forward(artlite_moe_layer* L, const void* x, in
   HostCtx* c = nullptr;
   if (T > 0 && y && xb <= PIN_MAX && CB + yb <= PIN_MAX) ART_TRY(host_ctx(&c, false));
   if (c && c->pins(xb, CB + yb)) {  // (through the thread's pinned buffers: one synchronization)
-    ART_TRY(check_ready(L));
     Drain drain{L->stream};
     std::memcpy(c->pin_in.p, x, xb);
     ART_TRY(launch_copy2(L->x.p, c->pin_in.p, xb, nullptr, nullptr, 0, nullptr, 0, L->stream));
     L->x_dtype = x_dtype;
     L->staged = T;
+    ART_TRY(check_ready(L));
     ART_TRY(run(L, T, nullptr));
     uint8_t* out = c->pin_out.as<uint8_t>();
     ART_TRY(launch_copy2(out + CB, L->y.p, yb, out, L->ctrl.p, CTRL_WORDS * 4, nullptr, 0, L->stream));

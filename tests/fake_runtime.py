@@ -24,18 +24,19 @@ from artlite_amd.moe.layer import TENSORS, MoELayer
 from artlite_amd.moe.plan import Plan, route
 BLOCK = dict(Q4_0=(32, 18), Q4_1=(32, 20), Q8_0=(32, 34), Q3_K=(256, 110), Q4_K=(256, 144), Q5_K=(256, 176),
              Q6_K=(256, 210), IQ4_NL=(32, 18), IQ4_XS=(256, 136))
-def layer(ready=True, **a):
-    L = MoELayer(**a)
+def upload(L, a):
     H, E, F, S = a["hidden"], a["n_experts"], a["expert_ffn"], a.get("shared_ffn", 0)
     def rows(n, cols, q): return n * (cols // BLOCK[q][0]) * BLOCK[q][1]
-    if ready:
-        sizes = dict(ffn_gate_inp=E * H * 4, ffn_gate_exps=rows(E * F, H, a["gate_type"]),
-                     ffn_up_exps=rows(E * F, H, a["gate_type"]), ffn_down_exps=rows(E * H, F, a["down_type"]))
-        if S:
-            q = a["shared_type"]
-            sizes.update(ffn_gate_shexp=rows(S, H, q), ffn_up_shexp=rows(S, H, q),
-                         ffn_down_shexp=rows(H, S, a.get("shared_down_type") or q))
-        for name, n in sizes.items(): L.upload(name, np.zeros(n, np.uint8))
+    sizes = dict(ffn_gate_inp=E * H * 4, ffn_gate_exps=rows(E * F, H, a["gate_type"]),
+                 ffn_up_exps=rows(E * F, H, a["gate_type"]), ffn_down_exps=rows(E * H, F, a["down_type"]))
+    if S:
+        q = a["shared_type"]
+        sizes.update(ffn_gate_shexp=rows(S, H, q), ffn_up_shexp=rows(S, H, q),
+                     ffn_down_shexp=rows(H, S, a.get("shared_down_type") or q))
+    for name, n in sizes.items(): L.upload(name, np.zeros(n, np.uint8))
+def layer(ready=True, **a):
+    L = MoELayer(**a)
+    if ready: upload(L, a)
     return L
 def names(T, x="bf16", **a):
     with layer(ready=False, max_tokens=T, **a) as L:

@@ -69,3 +69,16 @@ CALLS["route"]()
 CALLS["plan"]()
 assert hip.streams == 2
 """)
+
+
+def test_call_before_the_upload_stages_its_input(tmp_path: Path) -> None:
+    """layer(x) without its tensors is refused, and has staged x: once they are there, it runs."""
+    run_fake(tmp_path, """
+a = dict(hidden=1024, n_experts=8, top_k=2, expert_ffn=512, gate_type="Q8_0", down_type="Q8_0", max_tokens=64)
+L = layer(ready=False, **a)
+try: L(np.zeros((40, 1024), np.float32))
+except _hip.Error as e: assert "not uploaded" in str(e), e
+else: raise AssertionError
+upload(L, a)
+_hip.check(_hip.lib().artlite_moe_layer_run(L.handle, 40))
+""")
