@@ -589,9 +589,9 @@ int launch_t(const StreamArgs& a, bool dry, hipStream_t s) {
   const int cus = device_cus();
   if (!ok || cus <= 0) return fail(ARTLITE_EHIP, "streamed tiles: kernel set-up failed");
   int64_t grid = 0, entries = 0;
-  if (!stream_grid<QT, SWIGLU, WAVES, NC>(items, cus, grid, entries))
-    return fail(ARTLITE_EINVAL, "streamed tiles: %lld work items", (long long)items);
-  if (dry) return ARTLITE_OK;
+  const bool fits = stream_grid<QT, SWIGLU, WAVES, NC>(items, cus, grid, entries);
+  if (dry) return fits ? ARTLITE_OK : ARTLITE_EINVAL;
+  if (!fits) return fail(ARTLITE_EINVAL, "streamed tiles: %lld work items", (long long)items);
   k_stream<QT, SWIGLU, WAVES, NC><<<unsigned(grid), L::THREADS, L::LDS + size_t(entries) * L::ENTRY * 4, s>>>(a);
   ART_HIP(hipGetLastError());
   return ARTLITE_OK;
@@ -604,7 +604,7 @@ template <int QT, int NC>
 int launch_bm(const StreamArgs& a, bool dry, hipStream_t s) {
   constexpr int W = 2 * (SL<QT, true, 4, NC>::LDS + 2048) <= LDS_BYTES ? 4 : 8;
   if constexpr (NC == 4 && QT != ARTLITE_Q4_0 && QT != ARTLITE_Q4_K && QT != ARTLITE_Q8_0)
-    return fail(ARTLITE_EINVAL, "streamed tiles: %d rows of weight type %d", 16 * NC, QT);
+    return dry ? ARTLITE_EINVAL : fail(ARTLITE_EINVAL, "streamed tiles: %d rows of weight type %d", 16 * NC, QT);
   else
     return a.w[1] ? launch_t<QT, true, W, NC>(a, dry, s) : launch_t<QT, false, W, NC>(a, dry, s);
 }
@@ -632,6 +632,7 @@ bool stream_supported(int qtype, int K, int N) {
   }
 
 namespace {
+// (dry: whether a launch takes the items, as a status and no message)
 int by_type(const StreamArgs& a, bool dry, hipStream_t s) {
 #define ART_ST(QT) \
   return a.bm == 16   ? launch_bm<QT, 1>(a, dry, s)  \

@@ -82,3 +82,18 @@ else: raise AssertionError
 upload(L, a)
 _hip.check(_hip.lib().artlite_moe_layer_run(L.handle, 40))
 """)
+
+
+def test_last_error_outlives_a_pass(tmp_path: Path) -> None:
+    """Asking whether a launch takes a pass's items, and finding that it does not, leaves the thread's message alone."""
+    run_fake(tmp_path, """
+a = dict(hidden=1024, n_experts=1024, top_k=8, expert_ffn=4096, gate_type="Q4_0", down_type="Q4_0")
+with layer(ready=False, max_tokens=128 * 36, **a) as L:
+    try: L.upload("ffn_gate_inp", np.zeros(10, np.uint8))
+    except _hip.Error as e: said = str(e)
+    for pairs in (4, 33, 36):
+        L.stage(np.zeros((128 * pairs, 1024), np.uint16))
+        n = L.kernel_names()
+        assert not any("@stream64" in k for k in n), n
+        assert _hip.last_error() == said, (pairs, _hip.last_error())
+""")
