@@ -175,7 +175,7 @@ __global__ __launch_bounds__(DISPATCH_BLOCK) void k_scatter(DispatchBufs d, Plan
   const int t = int((p < d.P ? p : d.P - 1) / d.k);  // (pairs past P: the last pair's token, unused)
   const int base = d.table[int64_t(blockIdx.x) * d.E + (valid ? id : 0)];
   float2 f0 = {0.0f, 0.0f}, f1 = f0;
-  if (d.row_f[0]) f0 = d.row_f[0][t], f1 = d.row_f[1][t];
+  if (d.row_a) f0 = d.row_f[0][t], f1 = d.row_f[1][t];
   asm volatile("" : : "v"(base), "v"(f0.x), "v"(f0.y), "v"(f1.x), "v"(f1.y));
   // the lanes of this wave with the same expert (ballots over the id bits)
   uint64_t peers = __ballot(valid);
@@ -195,10 +195,8 @@ __global__ __launch_bounds__(DISPATCH_BLOCK) void k_scatter(DispatchBufs d, Plan
   d.slot[p] = dest;
   if (d.row_a) {  // (the prefill's per-row token and factors, gathered here rather than by a launch of their own)
     d.row_a[dest] = t;
-    if (d.row_f[0]) {
-      d.row_out[0][dest] = f0;
-      d.row_out[1][dest] = f1;
-    }
+    d.row_out[0][dest] = f0;
+    d.row_out[1][dest] = f1;
   }
   if (pl.pos) {  // the plan's row of this pair
     const int o = dest - d.offsets[id];
