@@ -17,7 +17,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize(("T", "E", "k"), [(1, 32, 2), (1023, 128, 8), (1025, 128, 8), (8191, 128, 4), (8193, 128, 4),
-                                           (40, 1000, 6)])
+                                           (40, 1000, 6),
+                                           # (several parts, whose first and last rows share cache lines)
+                                           (2100, 129, 8), (6001, 77, 5)])
 def test_route_sizes(T: int, E: int, k: int) -> None:
     lg = np.random.default_rng(T).standard_normal((T, E)).astype(np.float32)
     ids, w = MP.route(lg, k)
@@ -41,6 +43,7 @@ def test_route_overlapping_rows() -> None:
     _hip.check(_hip.lib().artlite_moe_route(_hip.ptr(flat, c.c_float), flat.size, T, row, per_col, pitch, E, 4, 0,
                                             _hip.ptr(ids, c.c_int32), _hip.ptr(w, c.c_float)))
     assert np.array_equal(ids, want[0])
+    np.testing.assert_allclose(w, want[1], rtol=1e-6)
 
 
 @pytest.mark.parametrize(("T", "k", "E"), [(3, 2, 8), (20000, 8, 64), (60000, 8, 64)])

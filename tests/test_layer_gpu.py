@@ -106,7 +106,9 @@ def check_layer(name: str, T: int, seed: int = 0) -> None:
                               (spec.H, spec.H, spec.shared_F)))
             a = x64 @ sg.T
             ys64 = (a / (1 + np.exp(-a)) * (x64 @ su.T)) @ sd.T
-            assert rel_l2(g.tap("y_shared"), ys64) < (1e-3 if prefill else max(tol, 1e-4)), name
+            # (on the streamed dense rows: x (in the gate and the up product) and h to 2^-17)
+            streamed = "shared_down@stream" in g.kernel_names()
+            assert rel_l2(g.tap("y_shared"), ys64) < (3 * 2.0**-17 if streamed else 1e-3 if prefill else max(tol, 1e-4)), name
         # output: the fp32 oracle and float64 math for the GPU's routing
         want = moe_ref.moe_ffn(x, ids, w, get) + layers.shared_out(layer, x)
         assert rel_l2(y, want) < 1e-3, (name, T, rel_l2(y, want))
