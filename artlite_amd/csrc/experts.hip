@@ -1,5 +1,5 @@
-// The experts' products over raw GGUF blocks on gfx950's MFMA, and the combine: the MFMA decode tiles (bf16, for
-// batches between the GEMV's and the prefill's; every Q4_K product), the prefill tiles (fp16, below), the combine.
+// The experts' products over raw GGUF blocks on gfx950's MFMA, and the combine: the MFMA decode tiles (bf16, for the shapes
+// that the prefill tiles and the GEMV do not take), the activations of the prefill tiles (fp16, below), the combine.
 //
 // MFMA decode tiles. Exactness of the operands: a block's integer codes are exact in bf16 -- Q4_0 as 128 + q and Q4_K as 128 + q
 // (a byte 0x43 above the nibble: bf16 128 + q), Q8_0 as 128 + q through an unsigned byte conversion -- and bf16

@@ -186,7 +186,7 @@ constexpr int stream_64(int qtype) {  // (0: no tiles of 64)
 }
 
 // A shared expert beside streamed routed ones: up to this many tokens on the streamed dense rows, whose launches take its
-// few weight rows 16 tokens at a time, past them on launches of the prefill tiles. (2816 wide, Q4_K, the layer at 64 / 128
+// few weight rows 16 tokens at a time, past them on launches of the prefill tiles of its own. (2816 wide, Q4_K, the layer at 64 / 128
 // / 256 / 320 tokens: 166 / 188 / 240 / 276 us against 223 / 235 / 280 / 289, in fp32 175 / 202 / 259 / 300 against 224 /
 // 233 / 281 / 289; 512 wide, Q8_0, 64 / 128 / 180 tokens: 76 / 83 / 87 against 113 / 120 / 123.)
 constexpr int64_t SHARED_STREAM = 256;
@@ -235,21 +235,24 @@ bool shared_streams(const artlite_moe_layer* L, int64_t T) {
 }
 
 // The kernels a forward pass of T tokens takes. Decode-sized passes (at most GEMV_BM pairs per expert on
-// average) run the experts on the VALU GEMV over XQ activations (it takes every block format); larger ones on the
-// fp16 MFMA prefill tiles (every block format: Q4_0, Q8_0, Q4_K from the file's bytes, the others through the prefill
-// layout), and where those do not take a product's shape (K below 320 or not a multiple of 64) on the MFMA decode
-// tiles over bf16 planes. (The GEMV takes widths of partial units in the formats of 32-value blocks: at 8 tokens of 64
-// experts 1408 wide the routed experts took 183 us on the prefill tiles, whose steps are as long for two rows of a tile
-// as for 32, and 47 us on the GEMV; at 5 tokens of 32 experts 2880 wide the layer 215 against 91 us.) Between
-// them and the prefill sizes the routed products stream (above).
+// average) run the experts on the VALU GEMV over XQ activations (it takes every block format); past them the routed
+// products stream (above), and larger passes run on the fp16 MFMA prefill tiles (every block format: Q4_0, Q8_0, Q4_K from
+// the file's bytes, the others through the prefill layout). Where the prefill tiles do not take a product's shape (K below
+// 320 or not a multiple of 64, tensors beyond their offsets) the routed experts of every size the GEMV does not take are on
+// the MFMA decode tiles over bf16 planes. A shared expert not on the GEMV and with no prefill launch is on the streamed
+// dense rows, which take any number of tokens (4096 tokens of 32 experts 768 wide with one of 256, Q8_0: 395 us, 532 with it
+// on the MFMA decode tiles), else on the MFMA decode tiles. (The GEMV takes widths of partial units in the formats of
+// 32-value blocks: at 8 tokens of 64 experts 1408 wide the routed experts took 183 us on the prefill tiles, whose steps are
+// as long for two rows of a tile as for 32, and 47 us on the GEMV; at 5 tokens of 32 experts 2880 wide the layer 218 against
+// 96 us.)
 struct Path {
   bool gemv;            // routed experts (gate / up and down) on the GEMV (XQ of x; tiles of GEMV_BM rows)
   bool shared_gemv;     // the shared expert on the GEMV
   bool prefill;         // routed experts on the prefill tiles
   int stream;           // ... their products by the streamed small tiles: their rows (16, 32 or 64), 0: not
   bool shared_prefill;  // the shared expert on the prefill tiles
-  bool shared_stream;   // the shared expert on the streamed small tiles (bf16 planes)
-  bool split;           // bf16 hi / lo planes of fp32 x needed (the MFMA decode tiles)
+  bool shared_stream;   // the shared expert on the streamed dense rows (bf16 planes)
+  bool split;           // bf16 hi / lo planes of fp32 x needed (the MFMA decode tiles, the streamed dense rows)
   bool quant;           // XQ of x needed (made by the router's launch)
   bool few_router;      // the router's launch of few tokens: a workgroup per expert and 16 tokens (and XQ of x)
   bool gemv_route;      // top k and dispatch in the gate / up GEMV's launch (each workgroup in its LDS)
@@ -771,8 +774,8 @@ extern "C" int artlite_moe_layer_create(const artlite_moe_desc* desc, artlite_mo
       return fail(ARTLITE_EINVAL, "moe layer: shared expert types %d / %d, width %d", d.shared_type,
                   d.shared_down_type, d.shared_ffn);
   }
-  // the MFMA decode tiles (every product between the GEMV's sizes and the prefill's, and every format the other two
-  // do not take) stage an A row's whole K in LDS: K up to 32 MAX_GROUPS
+  // the MFMA decode tiles, which take the products that no other path does, stage an A row's whole K in LDS: K up to 32
+  // MAX_GROUPS
   const int kmax = 32 * MAX_GROUPS;
   if (d.hidden > kmax || d.expert_ffn > kmax || d.shared_ffn > kmax)
     return fail(ARTLITE_EINVAL, "moe layer: H %d, F %d, shared F %d: at most %d each", d.hidden, d.expert_ffn,
@@ -810,8 +813,8 @@ extern "C" int artlite_moe_layer_create(const artlite_moe_desc* desc, artlite_mo
   L->gemv_ok = gemv_supported(d.gate_type, d.hidden, d.expert_ffn) &&
                gemv_supported(d.down_type, d.expert_ffn, d.hidden) &&
                ((d.hidden % 256 == 0 && d.expert_ffn % 256 == 0) || L->prefill_ok);
-  // (a shared expert beside routed ones of a partial unit stays on the MFMA decode tiles: its bf16 hi / lo planes hold
-  // x and h to 2^-17, XQ to 2^-16 of a group's largest, and its output is the layer's largest term)
+  // (a shared expert beside routed ones of a partial unit is on the streamed dense rows, not the GEMV: bf16 hi / lo planes
+  // hold x and h to 2^-17, XQ to 2^-16 of a group's largest, and its output is the layer's largest term)
   L->shared_gemv_ok = sq && d.hidden % 256 == 0 && d.expert_ffn % 256 == 0 && d.shared_ffn % 256 == 0 &&
                       gemv_supported(sq->id, d.hidden, d.shared_ffn) &&
                       gemv_supported(sdq->id, d.shared_ffn, d.hidden);

@@ -1,5 +1,5 @@
 // The streamed small tiles (stream.hip): the experts' grouped products for tiles of at most 64 rows over raw GGUF
-// blocks, on the prefill's fp16 activations, and the same for a few dense rows on bf16 (hi + lo) ones.
+// blocks, on the prefill's fp16 activations, and the same for dense rows on bf16 (hi + lo) ones.
 #pragma once
 
 #include "common.h"

@@ -465,8 +465,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((
   }
 }
 
-// The dense rows of a few tokens (the shared expert beside decode-sized routed ones) on bf16 planes: a product whose
-// items are too few for the device, so a workgroup takes 16 weight rows of gate and of up (plain: 32 rows) of a tile and
+// The dense rows of a shared expert beside decode-sized or streamed routed ones (a few to 256 tokens; any number where it has
+// no prefill tiles), on bf16 planes: at a few tokens a product whose items are too few for the device, so a workgroup takes 16 weight rows of gate and of up (plain: 32 rows) of a tile and
 // its 8 waves split K: wave w streams steps w, w + 8, ... of every row by DMA into its LDS slot, its activations come
 // from memory (L2) to registers, and the waves' sums meet in LDS, added in wave order by wave 0, which writes the
 // outputs. What bounds it is latency: a launch, two memory round trips, a step or two of products and the exchange
