@@ -37,14 +37,14 @@ CASES = [("cpu", 16), ("decode", 1), ("decode", 4), ("decode", 16), ("decode", 6
          # 320 and 160 experts past the GEMV's sizes (the MFMA decode tiles): the router's K in parts that the top-k
          # launch adds, eight and four logits a lane
          ("wide_e", 384), ("widek", 256)]
-# (passes on the MFMA decode tiles)
+# (passes with routed experts on the MFMA decode tiles)
 DTILE_CASES = {("dtiles", 96), ("wide_e", 384), ("widek", 256)}
 
 # Decode-sized passes (at most 4 pairs per expert on average, K a multiple of 256) take the GEMV over XQ activations:
 # int8 hi / lo planes per 32 values, |x - xq| <= max|x| / 65024 per group, so h (itself held in XQ) and the pair
 # outputs carry a few 1e-5 of relative error; the MFMA decode tiles' bf16 hi / lo planes, about 2^-17. Larger passes
-# take the prefill tiles' fp16 products: weights d (q - 8) and h rounded once to fp16 (2^-11 relative at most), a few
-# 1e-4 of relative error in h and the pair outputs.
+# take fp16 products: fp32 x and h rounded once to fp16 (2^-11 relative at most) and, on the prefill tiles past the streamed
+# ones, weights d (q - 8) too, a few 1e-4 of relative error in h and the pair outputs.
 GEMV_CASES = {("cpu", 16), ("decode", 1), ("decode", 4), ("decode", 16), ("decode", 64), ("mix_q8k", 16), ("mix_k8", 24),
               ("kmix", 16), ("q5km", 16), ("q5k", 24), ("kquants", 32), ("q6k", 24), ("mixtile", 16), ("iq4", 16),
               ("q41", 16), ("q3k", 16), ("widek", 40), ("widek", 16), ("topk20", 12), ("wide_e", 16)}
