@@ -10,9 +10,9 @@ namespace artlite {
 // rows of A (tokens for gate / up, pairs for down) per decode tile
 constexpr int GEMV_BM = 4;
 
-// XQ, the decode activations: each row of K values (K a multiple of 64) as units of 256 values (the last one's groups
-// past K are zeros), a unit as 8 groups of 32 and each group as two int8 planes, x ~ s (a + b / 256) with s = max |x| / 127 over the group. A
-// group's block is 16 dwords: plane a (8 dwords of 4 int8 in value order), then plane b. Per group three words:
+// XQ, the decode activations: each row of K values (K a multiple of 64) as units of 256 values (the last one's groups past
+// K are zeros), a unit as 8 groups of 32 and each group as two int8 planes, x ~ s (a + b / 256) with s = max |x| / 127 over
+// the group. A group's block is 16 dwords: plane a (8 dwords of 4 int8 in value order), then plane b. Per group three words:
 // s / 256 (fp32), the sum over the group of 256 a + b (int32), and s / 256 times that sum (fp32: the group's
 // dequantised sum). A group with a non-finite value has s = NaN; a group of zeros has s = 0.
 // A unit is 64 chunks of 4 dwords, chunk 16 p + r (p < 4, r < 16) = [dword r of group 2 p's block, dword r of group
